@@ -1,0 +1,80 @@
+"""The tiled MFMA GEMM of batches above 32 columns at its edges: last row tiles, last column tiles, every column-tile
+width, formats whose rows straddle 16-byte chunks, K other than the weight-stationary kernel's, unaligned outputs."""
+import numpy as np
+import pytest
+
+from oracle import dequant as dq
+from oracle import step as ost
+from tests._dev import down, empty, up
+from tests.conftest import rel_l2
+from vte_amd import synthetic as syn
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-3  # fp32 sums of fp16 activations (2.1e-4 with fp32 inputs rounded, fp16 results likewise)
+
+
+@pytest.mark.parametrize("fmt", ["q4_k", "q6_k"])
+@pytest.mark.parametrize("n,k,M,io", [(8960, 256, 33, "f32"), (8961, 512, 64, "f16"), (4100, 1536, 96, "f16f32"),
+                                      (1, 256, 97, "f16f32"), (33333, 256, 65, "f16"), (130, 768, 515, "f32"),
+                                      (17000, 512, 161, "f16f32")])
+def test_gemm_tiled(hip, K, fmt, n, k, M, io):
+    """vte_gemm_mfma above 32 columns, with bias, residual and scale when the results are fp16."""
+    rng = np.random.default_rng(n + M)
+    raw = syn.random_matrix(fmt, rng, n, k, balanced=True)
+    x = rng.standard_normal((M, k)).astype(np.float32 if io == "f32" else np.float16)
+    odt = np.float16 if io == "f16" else np.float32
+    y = empty(hip, (M, n), odt)
+    kw, bias, res = {}, None, None
+    if io == "f16":
+        bias, res = rng.standard_normal(n).astype(odt), rng.standard_normal((M, n)).astype(odt)
+        kw = dict(bias=up(hip, bias), residual=up(hip, res), residual_scale=0.5)
+    K.gemm_mfma(fmt, up(hip, x), up(hip, raw), y, M, k, n, in_dtype="f32" if io == "f32" else "f16",
+                out_dtype="f16" if io == "f16" else "f32", stream=hip.stream, **kw)
+    rows = np.unique(np.concatenate([np.arange(min(n, 150)), np.arange(max(0, n - 150), n)]))
+    ref = dq.gemv(fmt, raw.reshape(n, -1)[rows].reshape(-1), len(rows), k, x.astype(np.float32))
+    if io == "f16":
+        ref = dq.gemv_epilogue(ref, bias[rows], res[:, rows], 0.5)
+    got = down(y)[:, rows].astype(np.float64)
+    assert np.isfinite(got).all()
+    for m0 in range(0, M, 16):  # a wrong column tile cannot hide in the norm of the others
+        assert rel_l2(got[m0:m0 + 16], ref[m0:m0 + 16]) <= TOL, m0
+
+
+@pytest.mark.parametrize("k,ffn,B", [(256, 8200, 70), (512, 4099, 129), (1536, 9001, 33), (2048, 5000, 100)])
+def test_ffn_in_tiled(hip, K, k, ffn, B):
+    """Gate/up + SwiGLU: ragged last pairs and columns, rows of the output off 16-byte alignment."""
+    rng = np.random.default_rng(ffn)
+    wg, wu = (syn.random_matrix("q4_k", rng, ffn, k, balanced=True) for _ in range(2))
+    x = rng.standard_normal((B, k)).astype(np.float16)
+    out = empty(hip, (B, ffn), np.float16)
+    K.ffn_in(up(hip, x), None, 1e-6, up(hip, wg), up(hip, wu), "q4_k", out, B, k, ffn, stream=hip.stream)
+    g, u = (dq.gemv("q4_k", w, ffn, k, x.astype(np.float32)).astype(np.float16) for w in (wg, wu))
+    got, ref = down(out), ost.swiglu(g, u)
+    assert rel_l2(got, ref) <= TOL
+    assert rel_l2(got[-1], ref[-1]) <= TOL and rel_l2(got[:, -8:], ref[:, -8:]) <= TOL
+
+
+@pytest.mark.parametrize("fmt,k,n,M,splits", [("q4_k", 8960, 1536, 164, 5), ("q6_k", 2048, 1537, 300, 8),
+                                              ("q6_k", 8960, 1500, 200, 7), ("q4_k", 256, 9000, 512, 1)])
+def test_splitk_tiled(hip, K, fmt, k, n, M, splits):
+    """Split-K partial sums of the tiled form: the bits of the 32-column launches."""
+    import os
+    rng = np.random.default_rng(k + M)
+    raw = syn.random_matrix(fmt, rng, n, k, balanced=True)
+    x = rng.standard_normal((M, k)).astype(np.float16)
+    dx, dw = up(hip, x), up(hip, raw)
+
+    def run():
+        part = empty(hip, (splits, M, n), np.float32)
+        K.gemm_mfma_splitk(fmt, dx, dw, part, M, k, n, splits, stream=hip.stream)
+        return down(part)
+
+    got = run()
+    os.environ["VTE_MM_WS"] = "0"
+    try:
+        one = run()
+    finally:
+        del os.environ["VTE_MM_WS"]
+    assert np.array_equal(got.view(np.uint32), one.view(np.uint32))
+    ref = dq.gemv(fmt, raw, n, k, x.astype(np.float32))
+    assert rel_l2(got.sum(0, dtype=np.float64), ref) <= TOL

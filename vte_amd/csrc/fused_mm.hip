@@ -20,7 +20,7 @@
 #include <cstdlib>
 #include <cstring>
 
-#include "mfma_deq.h"
+#include "mm_tile.h"
 
 #define MM_MAX_SEG 3
 
@@ -177,8 +177,41 @@ __device__ __forceinline__ float mm_sum(float (*red)[RT][NT][4][64], int rr, int
 
 __device__ __forceinline__ float mm_bias(const __half* b, int row) { return b ? __half2float(b[row]) : 0.f; }
 
-// Epilogue of one C tile group: batch columns cb .. cb + mcount - 1 of the
-// launch (column m reads kv_offset[m] and writes row m of the outputs).
+// Epilogue of one output (row, batch column m of the launch: position
+// kv_offset[m], row m of the outputs) from its sum.
+__device__ __forceinline__ void mm_put(const MmPlan& P, const MmSeg& S, int row, int m, float sum) {
+    const __half v = __float2half(sum + mm_bias(S.bias, row));
+    if (S.mode == MM_VCACHE) {
+        const int pos = P.kv_offset[m];
+        P.v_cache[(size_t)m * P.kv_batch_stride + ((size_t)pos * P.n_kv + row / 128) * 128 + (row % 128)] = v;
+    } else {
+        S.out[(size_t)m * S.n_rows + row] = v;
+    }
+}
+// The same for a pair: gate row and up row `row`, or rows `row`, `row` + 64 of one head.
+__device__ __forceinline__ void mm_put_pair(const MmPlan& P, const MmSeg& S, int row, int m, float a, float b) {
+    if (S.mode == MM_SWIGLU) {
+        const float g = __half2float(__float2half(a)), u = __half2float(__float2half(b));
+        S.out[(size_t)m * S.n_rows + row] = __float2half(g / (1.0f + expf(-g)) * u);
+        return;
+    }
+    const float x1 = __half2float(__float2half(a + mm_bias(S.bias, row)));
+    const float x2 = __half2float(__float2half(b + mm_bias(S.bias, row + 64)));
+    const int pos = P.kv_offset[m], d = row & 127;
+    const float c = __half2float(P.rope_cos[(size_t)pos * 128 + d]);
+    const float sn = __half2float(P.rope_sin[(size_t)pos * 128 + d]);
+    const __half o1 = __float2half(x1 * c - x2 * sn), o2 = __float2half(x1 * sn + x2 * c);
+    if (S.mode == MM_ROPE_Q) {
+        S.out[(size_t)m * S.n_rows + row] = o1;
+        S.out[(size_t)m * S.n_rows + row + 64] = o2;
+    } else {
+        __half* kc = P.k_cache + (size_t)m * P.kv_batch_stride + ((size_t)pos * P.n_kv + row / 128) * 128;
+        kc[d] = o1;
+        kc[d + 64] = o2;
+    }
+}
+
+// Epilogue of a block's C tiles: batch columns cb .. cb + mcount - 1.
 template <int RT, int NT, int NW>
 __device__ __forceinline__ void mm_epilogue(const MmPlan& P, const MmTile& T, float (*red)[RT][NT][4][64], int cb,
                                             int mcount) {
@@ -186,48 +219,21 @@ __device__ __forceinline__ void mm_epilogue(const MmPlan& P, const MmTile& T, fl
     if (!mm_paired(S.mode)) {
         for (int o = threadIdx.x; o < 16 * RT * 16 * NT; o += blockDim.x) {
             const int rr = o / (16 * NT), mc = o % (16 * NT);
-            if (rr >= T.nvalid || mc >= mcount) continue;
-            const int row = T.j0 + rr, m = cb + mc;
-            const __half v = __float2half(mm_sum<RT, NT, NW>(red, rr, mc) + mm_bias(S.bias, row));
-            if (S.mode == MM_VCACHE) {
-                const int pos = P.kv_offset[m];
-                P.v_cache[(size_t)m * P.kv_batch_stride + ((size_t)pos * P.n_kv + row / 128) * 128 + (row % 128)] = v;
-            } else {
-                S.out[(size_t)m * S.n_rows + row] = v;
-            }
+            if (rr < T.nvalid && mc < mcount) mm_put(P, S, T.j0 + rr, cb + mc, mm_sum<RT, NT, NW>(red, rr, mc));
         }
         return;
     }
     for (int o = threadIdx.x; o < 8 * RT * 16 * NT; o += blockDim.x) {
         const int p = o / (16 * NT), mc = o % (16 * NT);
-        if (p >= T.nvalid || mc >= mcount) continue;
-        const float a = mm_sum<RT, NT, NW>(red, p, mc), b = mm_sum<RT, NT, NW>(red, p + 8 * RT, mc);
-        const int row = T.j0 + p, m = cb + mc;
-        if (S.mode == MM_SWIGLU) {
-            const float g = __half2float(__float2half(a)), u = __half2float(__float2half(b));
-            S.out[(size_t)m * S.n_rows + row] = __float2half(g / (1.0f + expf(-g)) * u);
-            continue;
-        }
-        const float x1 = __half2float(__float2half(a + mm_bias(S.bias, row)));
-        const float x2 = __half2float(__float2half(b + mm_bias(S.bias, row + 64)));
-        const int pos = P.kv_offset[m], d = row & 127;
-        const float c = __half2float(P.rope_cos[(size_t)pos * 128 + d]);
-        const float sn = __half2float(P.rope_sin[(size_t)pos * 128 + d]);
-        const __half o1 = __float2half(x1 * c - x2 * sn), o2 = __float2half(x1 * sn + x2 * c);
-        if (S.mode == MM_ROPE_Q) {
-            S.out[(size_t)m * S.n_rows + row] = o1;
-            S.out[(size_t)m * S.n_rows + row + 64] = o2;
-        } else {
-            __half* kc = P.k_cache + (size_t)m * P.kv_batch_stride + ((size_t)pos * P.n_kv + row / 128) * 128;
-            kc[d] = o1;
-            kc[d + 64] = o2;
-        }
+        if (p < T.nvalid && mc < mcount)
+            mm_put_pair(P, S, T.j0 + p, cb + mc, mm_sum<RT, NT, NW>(red, p, mc),
+                        mm_sum<RT, NT, NW>(red, p + 8 * RT, mc));
     }
 }
 
 // NW waves per block split K (6 for K = 1536: one super-block each).
 template <int RT, int NT, int NW>
-__global__ __launch_bounds__(64 * NW) void fused_mm_kernel(MmPlan P) {
+__global__ __launch_bounds__(64 * NW, RT == 2 && NT == 1 ? 4 : 1) void fused_mm_kernel(MmPlan P) {
     __shared__ float red[NW][RT][NT][4][64];
     __shared__ float xl[NW][NT * 128];  // minimum-term scratch per wave (q4_xmin)
     const MmTile T = mm_tile<RT>(P, blockIdx.x);
@@ -240,7 +246,8 @@ __global__ __launch_bounds__(64 * NW) void fused_mm_kernel(MmPlan P) {
 }
 
 
-// Weight-stationary form for long batches (prefill chunks), K = 6 super-blocks:
+// Weight-stationary form for batches above 32 columns with few row tiles, K = 6
+// super-blocks:
 // wave w decodes super-block w of its tile rows once, keeps the weight
 // operands in registers and runs them against the block's columns
 // [blockIdx.y * cols, ...) 16 * NT at a time; the next columns' activations
@@ -311,6 +318,80 @@ __global__ __launch_bounds__(64 * 6) void fused_mm_ws_kernel(MmPlan P, int cols)
     else mm_ws_body<6, RT, NT>(P, T, red, xl, c0, c1);
 }
 
+// Eight SwiGLU outputs of column m from the sums of eight gate and up rows.
+__device__ __forceinline__ half8_t mm_swiglu8(const float* g, const float* u) {
+    half8_t v;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float a = __half2float(__float2half(g[e])), b = __half2float(__float2half(u[e]));
+        v[e] = (_Float16)(a / (1.0f + expf(-a)) * b);
+    }
+    return v;
+}
+
+// Long batches (prompt chunks): the tiled main loop of mm_tile.h, each wave on
+// one 32-row tile (16 pairs, or 32 rows) of the plan.  SwiGLU launches store
+// through LDS in 16-byte pieces (2-byte stores of 16 neighbouring rows took
+// 13 of 78 us at 512 columns of 8960); the other modes store from the
+// accumulators, where a pair's two sums are in one lane.
+// WCH: chunks per staged weight row (9: Q4_K only, 14: some segment is Q6_K);
+// SW: the SwiGLU plan.
+template <int NT, int WCH, bool SW>
+__global__ __launch_bounds__(64 * MT_WAVES, 2) void fused_mm_tile_kernel(
+    MmPlan P, int row_blocks, int groups, int total) {
+    __shared__ MtLds<NT, WCH> L;
+    const MtTile bt = mt_tile(blockIdx.x, row_blocks, groups);
+    if (bt.rb >= row_blocks) return;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 15, grp = lane >> 4;
+    const int g = bt.rb * MT_WAVES + wv, c0 = bt.cg * 16 * NT;
+    const MmTile T = mm_tile<2>(P, min(g, total - 1));  // waves past the last tile repeat it and store nothing
+    const MmSeg& S = *T.S;
+    const auto row = [&](int r) { return mm_row<2>(T, r); };
+    floatx4_t acc[2][NT];
+    if (WCH == 9 || __builtin_amdgcn_readfirstlane(S.fmt) == 4)
+        mt_loop<4, NT, WCH>(P.x, P.K, c0, P.M, row, 0, P.K / QK_K, true, L, acc);
+    else
+        mt_loop<6, NT, WCH>(P.x, P.K, c0, P.M, row, 0, P.K / QK_K, true, L, acc);
+    if constexpr (SW) {
+        const MmSeg& S0 = P.seg[0];
+        const bool vec = S0.n_rows % 8 == 0 && (reinterpret_cast<uintptr_t>(S0.out) & 15) == 0;
+        mt_epilogue<NT, WCH>(L, acc, [&](int p0, int pc) {
+            for (int o = threadIdx.x; o < pc * 2 * MT_WAVES; o += 64 * MT_WAVES) {
+                const int mc = o / (2 * MT_WAVES), ch = o % (2 * MT_WAVES), m = c0 + p0 + mc;
+                const int j = bt.rb * 16 * MT_WAVES + 8 * ch;
+                if (m >= P.M || j >= S0.n_rows) continue;
+                const float* c = L.c + mc * MT_LDC + 32 * (ch >> 1) + 8 * (ch & 1);
+                const half8_t v = mm_swiglu8(c, c + 16);
+                _Float16* dst = reinterpret_cast<_Float16*>(S0.out) + (size_t)m * S0.n_rows + j;
+                if (vec) {
+                    *reinterpret_cast<half8_t*>(dst) = v;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (j + e < S0.n_rows) dst[e] = v[e];
+                }
+            }
+        });
+        return;
+    }
+    if (g >= total) return;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int m = c0 + nt * 16 + 4 * grp + i;
+            if (m >= P.M) continue;
+            if (!mm_paired(S.mode)) {
+#pragma unroll
+                for (int rt = 0; rt < 2; ++rt)
+                    if (16 * rt + col < T.nvalid) mm_put(P, S, T.j0 + 16 * rt + col, m, acc[rt][nt][i]);
+            } else if (col < T.nvalid) {
+                mm_put_pair(P, S, T.j0 + col, m, acc[0][nt][i], acc[1][nt][i]);
+            }
+        }
+}
+
 namespace vte {
 
 static MmSeg mm_seg(const void* w, const void* w2, void* out, const void* bias, int fmt, int n_rows, int mode, int K,
@@ -336,10 +417,49 @@ static int mm_env(const char* name, int dflt) {
     return v ? atoi(v) : dflt;
 }
 
+// Launch form of a batch of B columns, `tiles` 32-row tiles in all.  Above 32
+// columns at K = 6 super-blocks the tiled form where its blocks (of 32 columns
+// here) fill the chip, else the weight-stationary one, whose six waves each
+// take a super-block (q/k/v of 2048 rows, 40 / 256 / 512 columns: 7.9 / 13.3 /
+// 20.8 us against 18.9 / 19.1 / 22.4 tiled; gate/up of 17920 rows, 64 / 512
+// columns: 28.3 / 114 against 18.1 / 58.1); other K as in mt_beats_launches.
+// VTE_MM_WS=0 selects the 32-column launches for every batch.
+enum MmForm { MM_COLS32, MM_WS, MM_TILED };
+static MmForm mm_form(int B, int tiles, int K) {
+    if (B <= 32 || mm_env("VTE_MM_WS", 1) == 0) return MM_COLS32;
+    const int row_blocks = (tiles + MT_WAVES - 1) / MT_WAVES;
+    if (K == 6 * QK_K) return row_blocks * ((B + 31) / 32) < 258 ? MM_WS : MM_TILED;
+    return mt_beats_launches(row_blocks, B, K / QK_K, false) ? MM_TILED : MM_COLS32;
+}
+static hipError_t mm_run_tiled(MmPlan P, int B, hipStream_t st) {
+    int total = 0;
+    for (int s = 0; s < P.nseg; ++s) total += P.seg[s].tiles;
+    P.M = B;
+    const int rbs = (total + MT_WAVES - 1) / MT_WAVES, nt = mt_pick_nt(rbs, 1, B, device_cus());
+    const int groups = (B + 16 * nt - 1) / (16 * nt);
+    bool q6 = false;
+    for (int s = 0; s < P.nseg; ++s) q6 = q6 || P.seg[s].fmt != 4;
+#define MM_LAUNCH(NT_, W_, SW_) \
+    hipLaunchKernelGGL((fused_mm_tile_kernel<NT_, W_, SW_>), dim3(mt_grid(rbs, groups)), dim3(64 * MT_WAVES), 0, st, P, \
+                       rbs, groups, total)
+#define MM_LAUNCH_NT(W_, SW_)            \
+    do {                                 \
+        if (nt == 6) MM_LAUNCH(6, W_, SW_); \
+        else if (nt == 4) MM_LAUNCH(4, W_, SW_); \
+        else MM_LAUNCH(2, W_, SW_);      \
+    } while (0)
+    if (P.seg[0].mode == MM_SWIGLU) MM_LAUNCH_NT(9, true);  // gate/up: Q4_K
+    else if (q6) MM_LAUNCH_NT(14, false);
+    else MM_LAUNCH_NT(9, false);
+#undef MM_LAUNCH_NT
+#undef MM_LAUNCH
+    return hipGetLastError();
+}
+
 // Runs the plan over the batch: in chunks of 32 columns (one launch each), or
-// in one weight-stationary launch when the batch is longer than 32 columns.
+// in one weight-stationary launch.
 template <int RT>
-static hipError_t mm_run(MmPlan P, int B, size_t out_ld_elems[MM_MAX_SEG], hipStream_t st) {
+static hipError_t mm_run(MmPlan P, int B, MmForm form, size_t out_ld_elems[MM_MAX_SEG], hipStream_t st) {
     int total = 0;
     for (int s = 0; s < P.nseg; ++s) total += P.seg[s].tiles;
     const __half* x0 = P.x;
@@ -348,7 +468,7 @@ static hipError_t mm_run(MmPlan P, int B, size_t out_ld_elems[MM_MAX_SEG], hipSt
     for (int s = 0; s < P.nseg; ++s) out0[s] = P.seg[s].out;
     __half* kc0 = P.k_cache;
     __half* vc0 = P.v_cache;
-    if constexpr (RT == 4) if (B > 32 && P.K == 6 * QK_K && mm_env("VTE_MM_WS", 1)) {
+    if constexpr (RT == 4) if (form == MM_WS) {
         // 64 rows per block, 16 columns at a time: one block per CU
         const int g = ws_column_groups(total, B, device_cus());
         const int cols = ((B + 31) / 32 + g - 1) / g * 32, gy = (B + cols - 1) / cols;
@@ -356,7 +476,7 @@ static hipError_t mm_run(MmPlan P, int B, size_t out_ld_elems[MM_MAX_SEG], hipSt
         hipLaunchKernelGGL((fused_mm_ws_kernel<RT, 1>), dim3(total, gy), dim3(64 * 6), 0, st, P, cols);
         return hipGetLastError();
     }
-    if constexpr (RT <= 2) if (B > 32 && P.K == 6 * QK_K && mm_env("VTE_MM_WS", 1)) {
+    if constexpr (RT <= 2) if (form == MM_WS) {
         // two 6-wave blocks fit per CU
         const int g = ws_column_groups(total, B, 2 * device_cus());
         const int cols = ((B + 31) / 32 + g - 1) / g * 32, gy = (B + cols - 1) / cols;
@@ -394,9 +514,10 @@ hipError_t qkv_mm(const void* xn, const void* wq, const void* q_bias, int fmt_q,
                   int fmt_k, const void* wv, const void* v_bias, int fmt_v, void* q_out, void* k_cache, void* v_cache,
                   const int* kv_offset, int kv_batch_stride, const void* rope_cos, const void* rope_sin, int B, int K,
                   int n_q, int n_kv, hipStream_t st) {
-    // 64 rows per block from 129 columns (2048-token prefill in chunks of 512:
+    const MmForm form = mm_form(B, (n_q + 2 * n_kv) * 4, K);
+    // weight-stationary: 64 rows per block from 129 columns (2048-token prefill in chunks of 512:
     // 38.5 -> 37.2 ms; chunks of 64-128 are faster with 16)
-    const int RT = mm_env("VTE_MM_RT_QKV", B > 128 ? 4 : 1);
+    const int RT = form == MM_TILED ? 2 : mm_env("VTE_MM_RT_QKV", form == MM_WS && B > 128 ? 4 : 1);
     MmPlan P;
     memset(&P, 0, sizeof(P));
     P.K = K;
@@ -412,8 +533,11 @@ hipError_t qkv_mm(const void* xn, const void* wq, const void* q_bias, int fmt_q,
     P.v_cache = (__half*)v_cache;
     P.kv_batch_stride = kv_batch_stride;
     P.n_kv = n_kv;
+    if (form == MM_TILED) return mm_run_tiled(P, B, st);
     size_t ld[MM_MAX_SEG] = {(size_t)n_q * 128, 0, 0};
-    return RT == 4 ? mm_run<4>(P, B, ld, st) : RT == 2 ? mm_run<2>(P, B, ld, st) : mm_run<1>(P, B, ld, st);
+    return RT == 4   ? mm_run<4>(P, B, form, ld, st)
+           : RT == 2 ? mm_run<2>(P, B, form, ld, st)
+                     : mm_run<1>(P, B, form, ld, st);
 }
 
 // out [B][ffn] = fp16(silu(W_gate xn) * (W_up xn)) for RMSNorm-ed fp16 xn [B][K].
@@ -421,22 +545,21 @@ hipError_t gate_up_mm(const void* xn, const void* w_gate, const void* w_up, int 
                       hipStream_t st) {
     // 16 gate/up pairs per block (half the blocks of 8, activations read half
     // as often); 24 for 17-32 columns (measured: batch 32 2.26 -> 2.18 ms per
-    // step, batch 8-16 slightly slower); 32 in the weight-stationary form above
-    // 32 columns (one block per CU, but each activation chunk serves twice
-    // the rows: 2048-token prefill 51.9 -> 47.9 ms)
-    int RT = mm_env("VTE_MM_RT_FFN", B > 32 ? 4 : B > 16 ? 3 : 2);
-    if (B > 32 && RT == 3) RT = 2;
+    // step, batch 8-16 slightly slower); 32 in the weight-stationary form
+    const MmForm form = mm_form(B, (ffn + 15) / 16, K);
+    const int RT = form == MM_TILED ? 2 : mm_env("VTE_MM_RT_FFN", form == MM_WS ? 4 : B > 16 ? 3 : 2);
     MmPlan P;
     memset(&P, 0, sizeof(P));
     P.K = K;
     P.x = (const __half*)xn;
     P.seg[0] = mm_seg(w_gate, w_up, out, nullptr, fmt, ffn, MM_SWIGLU, K, RT);
     P.nseg = 1;
+    if (form == MM_TILED) return mm_run_tiled(P, B, st);
     size_t ld[MM_MAX_SEG] = {(size_t)ffn, 0, 0};
-    return RT == 4   ? mm_run<4>(P, B, ld, st)
-           : RT == 3 ? mm_run<3>(P, B, ld, st)
-           : RT == 2 ? mm_run<2>(P, B, ld, st)
-                     : mm_run<1>(P, B, ld, st);
+    return RT == 4   ? mm_run<4>(P, B, form, ld, st)
+           : RT == 3 ? mm_run<3>(P, B, form, ld, st)
+           : RT == 2 ? mm_run<2>(P, B, form, ld, st)
+                     : mm_run<1>(P, B, form, ld, st);
 }
 
 }  // namespace vte

@@ -4,8 +4,8 @@
 //
 // Same contract as the GEMV (vte/compiler/templates/rdna/gemv_q4k.hip.template:56-168);
 // the reference re-reads W once per batch row (grid.y = batch), this kernel
-// reads it once per 32-column batch tile (and the weight-stationary split-K
-// form once per column group of up to hundreds of columns).
+// reads it once per 32-column batch tile (above 32 columns once per column
+// group of up to 128, mm_tile.h).
 //
 // Design:
 //  * v_mfma_f32_16x16x32_f16 with exact integer weight operands and the
@@ -19,7 +19,7 @@
 #include <cstdlib>
 #include <type_traits>
 
-#include "mfma_deq.h"
+#include "mm_tile.h"
 
 // Body of one block: row tile blockIdx.x, split `split` of `nsplit` (split-K
 // partial sums at y + split * split_stride).
@@ -102,7 +102,7 @@ __device__ __forceinline__ void gemm_mfma_body(const TI* __restrict__ x, const u
 
 // NW waves per block split K (6 when K = 1536: one super-block each).
 template <typename TI, typename TO, int FMT, int RT, int NT, int NW = MF_WAVES>
-__global__ __launch_bounds__(64 * NW) void gemm_mfma_kernel(const TI* __restrict__ x, const uint8_t* __restrict__ w,
+__global__ __launch_bounds__(64 * NW, RT == 2 && NT == 1 ? 4 : 1) void gemm_mfma_kernel(const TI* __restrict__ x, const uint8_t* __restrict__ w,
                                                         TO* __restrict__ y, int M, int K, int N,
                                                         const TO* __restrict__ bias, const TO* __restrict__ residual,
                                                         float rs, size_t split_stride) {
@@ -148,7 +148,7 @@ extern "C" __global__ __launch_bounds__(64 * MF_WAVES) void gemm_q6k_mfma_kernel
 }
 
 
-// Weight-stationary split-K for long batches (prefill chunks): as
+// Weight-stationary split-K for batches above 32 columns with few row tiles: as
 // gemm_mfma_kernel with fp16 activations and fp32 partial sums, when no wave
 // owns more than one super-block of its block's range.  Each wave dequantises
 // its super-block of the 16 tile rows once and runs it against the block's
@@ -232,6 +232,49 @@ __global__ __launch_bounds__(64 * MF_WAVES) void gemm_ws_splitk_kernel(const __h
         }
         __syncthreads();
     }
+}
+
+// More than 32 columns (prompt chunks): the tiled main loop of mm_tile.h; grid
+// (row blocks x column groups, splits), split s writes its sums at
+// y + s * split_stride.
+template <typename TI, typename TO, int FMT, int NT>
+__global__ __launch_bounds__(64 * MT_WAVES, 2) void gemm_tile_kernel(
+    const TI* __restrict__ x, const uint8_t* __restrict__ w, TO* __restrict__ y, int M, int K, int N,
+    const TO* __restrict__ bias, const TO* __restrict__ residual, float rs, size_t split_stride, int row_blocks,
+    int groups) {
+    constexpr int WCH = MtRaw<FMT>::CHUNKS;
+    __shared__ MtLds<NT, WCH> L;
+    const MtTile bt = mt_tile(blockIdx.x, row_blocks, groups);
+    if (bt.rb >= row_blocks) return;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row0 = bt.rb * MT_ROWS, c0 = bt.cg * 16 * NT;
+    const int n_sb = K / QK_K, split = blockIdx.y, splits = gridDim.y;
+    const size_t row_bytes = (size_t)n_sb * MtRaw<FMT>::BPB;
+    const auto row = [&](int r) { return w + (size_t)min(row0 + 32 * wv + r, N - 1) * row_bytes; };
+    floatx4_t acc[2][NT];
+    mt_loop<FMT, NT, WCH>(x, K, c0, M, row, (n_sb * split) / splits, (n_sb * (split + 1)) / splits, FMT == 4, L, acc);
+    y += split * split_stride;
+    // four rows of a column at a time (one vector store where the rows of y allow it)
+    const bool vec = N % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & (4 * sizeof(TO) - 1)) == 0 && bias == nullptr &&
+                     residual == nullptr;
+    mt_epilogue<NT, WCH>(L, acc, [&](int p0, int pc) {
+        for (int o = threadIdx.x; o < pc * (MT_ROWS / 4); o += 64 * MT_WAVES) {
+            const int mc = o / (MT_ROWS / 4), r = 4 * (o % (MT_ROWS / 4)), m = c0 + p0 + mc;
+            if (m >= M || row0 + r >= N) continue;
+            const float4 v = *reinterpret_cast<const float4*>(L.c + mc * MT_LDC + r);
+            const float s[4] = {v.x, v.y, v.z, v.w};
+            if (vec) {
+                TO t[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) st_act<TO>(t + e, s[e] * rs);
+                __builtin_memcpy(__builtin_assume_aligned(y + (size_t)m * N + row0 + r, 4 * sizeof(TO)), t, sizeof(t));
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (row0 + r + e < N) gemv_store<TO>(y, bias, residual, rs, row0 + r + e, m, N, s[e]);
+            }
+        }
+    });
 }
 
 // ---------------------------------------------------------------------------
@@ -434,9 +477,35 @@ static hipError_t launch_stream(const void* x, const void* w, void* y, int M, in
     return hipSuccess;
 }
 
+// true when the environment variable is set to 0 (switches a launch form off)
+static bool getenv_off(const char* name) {
+    const char* v = getenv(name);
+    return v != nullptr && atoi(v) == 0;
+}
+
+// One tiled launch (more than 32 columns), `splits` shares of K.
+template <typename TI, typename TO, int FMT>
+static hipError_t launch_tiled(const TI* x, const void* w, TO* y, int M, int K, int N, const TO* bias,
+                               const TO* residual, float rs, int splits, hipStream_t st) {
+    const int rbs = (N + MT_ROWS - 1) / MT_ROWS;
+    const int nt = mt_pick_nt(rbs, splits, M, device_cus()), groups = (M + 16 * nt - 1) / (16 * nt);
+    const size_t ss = (size_t)M * N;
+#define MT_LAUNCH(NT_)                                                                                         \
+    hipLaunchKernelGGL((gemm_tile_kernel<TI, TO, FMT, NT_>), dim3(mt_grid(rbs, groups), splits), dim3(64 * MT_WAVES), \
+                       0, st, x, (const uint8_t*)w, y, M, K, N, bias, residual, rs, ss, rbs, groups)
+    if (nt == 6) MT_LAUNCH(6);
+    else if (nt == 4) MT_LAUNCH(4);
+    else MT_LAUNCH(2);
+#undef MT_LAUNCH
+    return hipGetLastError();
+}
+
 template <typename TI, typename TO, int FMT>
 static hipError_t launch_mfma(const void* x, const void* w, void* y, int M, int K, int N, const void* bias,
                               const void* residual, float rs, hipStream_t st) {
+    if (M > 32 && mt_beats_launches((N + MT_ROWS - 1) / MT_ROWS, M, K / QK_K, sizeof(TI) == 4) && !getenv_off("VTE_MM_WS"))
+        return launch_tiled<TI, TO, FMT>((const TI*)x, w, (TO*)y, M, K, N, (const TO*)bias, (const TO*)residual, rs, 1,
+                                         st);
     if (K == GS_K && N >= 16384 && gs_lds_ok(M)) return launch_stream<TI, TO, FMT>(x, w, y, M, N, bias, residual, rs, st);
     const bool tall = N >= 4096;
     for (int m0 = 0; m0 < M; m0 += 32) {
@@ -461,32 +530,29 @@ static hipError_t launch_mfma(const void* x, const void* w, void* y, int M, int 
 // super-blocks of dequant(W[n, k]) * x[m, k]; no bias, scale or residual (the
 // consumer adds the splits).  Splits multiply the blocks of a short-and-wide
 // problem (down projection: K = 8960, N = 1536) so the whole chip streams W.
-// true when the environment variable is set to 0 (switches a launch form off)
-static bool getenv_off(const char* name) {
-    const char* v = getenv(name);
-    return v != nullptr && atoi(v) == 0;
-}
-
 template <int FMT>
 static hipError_t launch_splitk(const void* x, const void* w, float* part, int M, int K, int N, int splits,
                                 hipStream_t st) {
     const size_t ss = (size_t)M * N;
     const int n_sb = K / QK_K;
     if (M > 32 && (n_sb + splits - 1) / splits <= MF_WAVES && !getenv_off("VTE_MM_WS")) {
-        // one launch; two 8-wave blocks fit per CU
-        if (getenv_off("VTE_MM_WS_RT4")) {  // 16 rows per block, 32 columns at a time
-            const int tiles = (N + 15) / 16;
-            const int g = ws_column_groups(tiles * splits, M, 2 * device_cus());
-            const int cols = ((M + 31) / 32 + g - 1) / g * 32, gz = (M + cols - 1) / cols;
-            hipLaunchKernelGGL((gemm_ws_splitk_kernel<FMT, 1, 2>), dim3(tiles, splits, gz), dim3(64 * MF_WAVES), 0,
-                               st, (const __half*)x, (const uint8_t*)w, part, M, K, N, ss, cols);
-        } else {  // 64 rows per block, 16 columns at a time: each activation chunk serves 4x the rows
-            const int tiles = (N + 63) / 64;
-            const int g = ws_column_groups(tiles * splits, M, device_cus());
-            const int cols = ((M + 31) / 32 + g - 1) / g * 32, gz = (M + cols - 1) / cols;
-            hipLaunchKernelGGL((gemm_ws_splitk_kernel<FMT, 4, 1>), dim3(tiles, splits, gz), dim3(64 * MF_WAVES), 0,
-                               st, (const __half*)x, (const uint8_t*)w, part, M, K, N, ss, cols);
-        }
+        // The tiled form from 43 blocks (of 32 columns) per super-block of a
+        // split, which it takes one after another (2.7 us each) where this form
+        // gives each a wave: 8960 -> 1536 in 5 splits, 128 / 256 / 512 columns,
+        // Q6_K 24.7 / 35.7 / 58.0 us weight-stationary against 21.2 / 27.3 / 34.6
+        // tiled, Q4_K 19.6 / 31.3 / 55.2 against 19.9 / 27.8 / 34.9 (64 columns:
+        // 13.8 against 19.1); 1536 -> 1536 in 2 splits, 128 / 256 / 512 columns,
+        // 11.1 / 16.0 / 24.9 against 11.4 / 12.3 / 15.4 (with the add + norm launch).
+        const int tb = (N + MT_ROWS - 1) / MT_ROWS * splits * ((M + 31) / 32);
+        if (tb >= 43 * ((n_sb + splits - 1) / splits))
+            return launch_tiled<__half, float, FMT>((const __half*)x, w, part, M, K, N, nullptr, nullptr, 1.f, splits,
+                                                    st);
+        // 64 rows per block, 16 columns at a time: each activation chunk serves 4x the rows
+        const int tiles = (N + 63) / 64;
+        const int g = ws_column_groups(tiles * splits, M, device_cus());
+        const int cols = ((M + 31) / 32 + g - 1) / g * 32, gz = (M + cols - 1) / cols;
+        hipLaunchKernelGGL((gemm_ws_splitk_kernel<FMT, 4, 1>), dim3(tiles, splits, gz), dim3(64 * MF_WAVES), 0, st,
+                           (const __half*)x, (const uint8_t*)w, part, M, K, N, ss, cols);
         return hipGetLastError();
     }
     for (int m0 = 0; m0 < M; m0 += 32) {

@@ -136,33 +136,34 @@ struct Q4Ops {
     float d, dmin;
 };
 
-__device__ __forceinline__ void q6_exact_operands(const Q6Raw& r, int grp, Q6Ops& o) {
-    o.d = h2f_bits(r.d);
+// Operand of k-step t.
+__device__ __forceinline__ half8_t q6_step_operand(const Q6Raw& r, int t, int grp) {
     const uint32_t la[4] = {r.la.x, r.la.y, r.la.z, r.la.w};
     const uint32_t lb[4] = {r.lb.x, r.lb.y, r.lb.z, r.lb.w};
     const uint32_t hq[4] = {r.hq.x, r.hq.y, r.hq.z, r.hq.w};
     const uint64_t sc = ((uint64_t)r.sc.y << 32) | r.sc.x;
-    const int j = grp & 1;
+    const int q = t >> 1, w0 = 2 * (t & 1);  // quarter; first code word of the step's 8 codes
+    uint32_t u[2];
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-        const int q = t >> 1, w0 = 2 * (t & 1);  // quarter; first code word of the step's 8 codes
-        uint32_t u[2];
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const uint32_t l = (q & 1) ? lb[w0 + e] : la[w0 + e];
-            const uint32_t nib = (q < 2) ? (l & 0x0F0F0F0Fu) : ((l >> 4) & 0x0F0F0F0Fu);
-            u[e] = nib | (((hq[w0 + e] >> (2 * q)) & 0x03030303u) << 4);
-        }
-        const float scq = (float)(int8_t)((sc >> (8 * (2 * q + j))) & 0xFF);
-        // (1024 + u) - 1056 = u - 32 exactly, then one multiply by the integer scale
-        H8 v;
-        bytes_to_f16magic(u[0], v.u[0], v.u[1]);
-        bytes_to_f16magic(u[1], v.u[2], v.u[3]);
-        const half2_t off = splat2(-1056.0f), s2 = splat2(scq);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v.h2[i] = (v.h2[i] + off) * s2;
-        o.w[t] = v.v;
+    for (int e = 0; e < 2; ++e) {
+        const uint32_t l = (q & 1) ? lb[w0 + e] : la[w0 + e];
+        const uint32_t nib = (q < 2) ? (l & 0x0F0F0F0Fu) : ((l >> 4) & 0x0F0F0F0Fu);
+        u[e] = nib | (((hq[w0 + e] >> (2 * q)) & 0x03030303u) << 4);
     }
+    const float scq = (float)(int8_t)((sc >> (8 * (2 * q + (grp & 1)))) & 0xFF);
+    // (1024 + u) - 1056 = u - 32 exactly, then one multiply by the integer scale
+    H8 v;
+    bytes_to_f16magic(u[0], v.u[0], v.u[1]);
+    bytes_to_f16magic(u[1], v.u[2], v.u[3]);
+    const half2_t off = splat2(-1056.0f), s2 = splat2(scq);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v.h2[i] = (v.h2[i] + off) * s2;
+    return v.v;
+}
+__device__ __forceinline__ void q6_exact_operands(const Q6Raw& r, int grp, Q6Ops& o) {
+    o.d = h2f_bits(r.d);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) o.w[t] = q6_step_operand(r, t, grp);
 }
 
 // Q4_K: the header and the lane's two 16-byte code chunks; operands for the
@@ -175,35 +176,62 @@ __device__ __forceinline__ void q4_raw_load(const uint8_t* blk, int grp, Q4Raw& 
     r.q0 = *reinterpret_cast<const uint4*>(blk + 16 + 16 * grp);
     r.q1 = *reinterpret_cast<const uint4*>(blk + 16 + 16 * (grp + 4));
 }
+// Byte b of u (< 256) as a splat fp16 pair, exactly.
+__device__ __forceinline__ half2_t byte_splat(uint32_t u, int b) {
+    const uint32_t v = __builtin_amdgcn_perm(0x64646464u, u, 0x04000400u + 0x00010001u * (uint32_t)b);
+    return __builtin_bit_cast(half2_t, v) + splat2(-1024.0f);
+}
+// The eight 6-bit scales of a Q4_K header, four to a word (get_scale_min_k4 on
+// all bytes at once), and its eight minima.
+__device__ __forceinline__ void q4_scale_words(const uint4& h, uint32_t (&sc)[2]) {
+    sc[0] = h.y & 0x3F3F3F3Fu;
+    sc[1] = (h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u);
+}
+__device__ __forceinline__ void q4_min_words(const uint4& h, uint32_t (&mn)[2]) {
+    mn[0] = h.z & 0x3F3F3F3Fu;
+    mn[1] = ((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u);
+}
+// Q4Ops::mins of a lane.
+__device__ __forceinline__ half8_t q4_mins(const uint4& h, int grp) {
+    uint32_t mn[2];
+    q4_min_words(h, mn);
+    H8 v;
+    bytes_to_f16magic(grp < 2 ? mn[0] : 0u, v.u[0], v.u[1]);
+    bytes_to_f16magic(grp < 2 ? mn[1] : 0u, v.u[2], v.u[3]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v.h2[i] = v.h2[i] + splat2(-1024.0f);
+    return v.v;
+}
+// Operand of the k-step that takes nibble `part`, half `e` of code chunk qc.
+__device__ __forceinline__ half8_t q4_step_operand(const uint4& qc, int part, int e, half2_t s2, half2_t c2) {
+    const uint32_t wa = e == 0 ? qc.x : qc.z, wb = e == 0 ? qc.y : qc.w;
+    const uint32_t u0 = part ? ((wa >> 4) & 0x0F0F0F0Fu) : (wa & 0x0F0F0F0Fu);
+    const uint32_t u1 = part ? ((wb >> 4) & 0x0F0F0F0Fu) : (wb & 0x0F0F0F0Fu);
+    return codes8(u0, u1, s2, c2);
+}
 template <bool XM>
 __device__ __forceinline__ void q4_exact_operands(const Q4Raw& r, int grp, Q4Ops& o) {
     o.d = h2f_bits(r.h.x);
     o.dmin = h2f_bits(r.h.x >> 16);
-    Q4KLaneInts s[2];
-    s[0] = q4k_lane_ints(r.h, grp >> 1);
-    s[1] = q4k_lane_ints(r.h, 2 + (grp >> 1));
+    uint32_t sc[2];
+    q4_scale_words(r.h, sc);
+    const int b0 = 2 * (grp >> 1);  // byte of the lane's first sub-block in either word
     if constexpr (!XM) {
-        o.mnb = s[0].mn0 | (s[0].mn1 << 8) | (s[1].mn0 << 16) | (s[1].mn1 << 24);
+        uint32_t mn[2];
+        q4_min_words(r.h, mn);
+        o.mnb = __builtin_amdgcn_perm(mn[1], mn[0], 0x05040100u + 0x02020202u * (uint32_t)(grp >> 1));
     } else {
-        half8_t mv;
+        o.mins = q4_mins(r.h, grp);
+    }
 #pragma unroll
-        for (int mb = 0; mb < 4; ++mb) {
-            const Q4KLaneInts v = q4k_lane_ints(r.h, mb);
-            mv[2 * mb] = grp < 2 ? (_Float16)(float)v.mn0 : (_Float16)0.0f;
-            mv[2 * mb + 1] = grp < 2 ? (_Float16)(float)v.mn1 : (_Float16)0.0f;
+    for (int ci = 0; ci < 2; ++ci)
+#pragma unroll
+        for (int part = 0; part < 2; ++part) {
+            const half2_t s2 = byte_splat(sc[ci], b0 + part), c2 = s2 * splat2(-1024.0f);  // exact: sc <= 63
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                o.w[4 * ci + 2 * part + e] = q4_step_operand(ci == 0 ? r.q0 : r.q1, part, e, s2, c2);
         }
-        o.mins = mv;
-    }
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-        const int ci = t >> 2, part = (t >> 1) & 1, e = t & 1;
-        const uint4 qc = ci == 0 ? r.q0 : r.q1;
-        const uint32_t wa = e == 0 ? qc.x : qc.z, wb = e == 0 ? qc.y : qc.w;
-        const uint32_t u0 = part ? ((wa >> 4) & 0x0F0F0F0Fu) : (wa & 0x0F0F0F0Fu);
-        const uint32_t u1 = part ? ((wb >> 4) & 0x0F0F0F0Fu) : (wb & 0x0F0F0F0Fu);
-        const float sc = (float)(part ? s[ci].sc1 : s[ci].sc0);
-        o.w[t] = codes8(u0, u1, splat2(sc), splat2(-1024.0f * sc));
-    }
 }
 
 // Sub-block sums of the activations of one super-block, X[m][j] = sum of
@@ -317,8 +345,8 @@ __device__ __forceinline__ void sb_mfma(const Q4Ops& o, const half8_t (&bx)[8][N
     for (int nt = 0; nt < NT; ++nt) aw[nt] = am[nt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
-        const _Float16 m = (_Float16)(float)((o.mnb >> (8 * (t >> 1))) & 0xFFu);
-        const half8_t mv = {m, m, m, m, m, m, m, m};
+        const half2_t m = byte_splat(o.mnb, t >> 1);
+        const half8_t mv = {m[0], m[1], m[0], m[1], m[0], m[1], m[0], m[1]};
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
             aw[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bx[t][nt], o.w[t], aw[nt], 0, 0, 0);
