@@ -297,3 +297,33 @@ def test_prompt_columns_sharing_one_cache(hip, K, B, start, split, dtype):
     for b in (0, B // 2, B - 1):
         ref = attention_ref(q[b].astype(odt).astype(np.float32), kc1[0], vc1[0], int(offsets[b]) + 1, SCALE)
         assert rel_l2(got[b].astype(np.float32), ref) <= TOL, b
+
+
+@pytest.mark.parametrize("B,offsets,n_q,n_kv,split,dtype", [
+    (65, "run", 12, 2, 128, "f16"), (130, "run", 7, 1, 128, "f32"), (200, "any", 28, 4, 128, "f16"),
+    (96, "first", 2, 2, 512, "f16"), (513, "run", 4, 1, 32, "f32"), (70, "last", 16, 2, 1024, "f16")])
+def test_prompt_chunk_attention(hip, K, B, offsets, n_q, n_kv, split, dtype):
+    """More than 64 columns of one cache (the 64-row blocks with shared K/V tiles): consecutive, arbitrary, all-first
+    and repeated-last positions, every GQA packing, one and several token shares; cache rows past the longest
+    column hold NaN and must not be read into any result."""
+    rng = np.random.default_rng(B)
+    max_seq = 1000
+    q = rng.standard_normal((B, n_q, D)).astype(np.float32 if dtype == "f32" else np.float16)
+    kc, vc = (rng.standard_normal((max_seq, n_kv, D)).astype(np.float16) for _ in range(2))
+    off = {"run": np.arange(300, 300 + B), "any": rng.integers(0, 900, B), "first": np.zeros(B, int),
+           "last": np.minimum(np.arange(B) + 930, 985)}[offsets].astype(np.int32)
+    kc[off.max() + 1:] = np.nan
+    vc[off.max() + 1:] = np.nan
+    ms = (max_seq + split - 1) // split
+    pm, pl = empty(hip, (B, n_q, ms), np.float32), empty(hip, (B, n_q, ms), np.float32)
+    po, out = empty(hip, (B, n_q, ms, D), np.float32), empty(hip, (B, n_q, D), q.dtype)
+    K.attn_split_kv(up(hip, q), up(hip, kc), up(hip, vc), pm, pl, po, out, B, n_q, n_kv, D, SCALE, up(hip, off), 0,
+                    split, ms, dtype=dtype, stream=hip.stream)
+    got = down(out).astype(np.float64)
+    for b in range(0, B, 1 if B < 100 else 7):
+        n = int(off[b]) + 1
+        for h in range(n_q):
+            s = kc[:n, h // (n_q // n_kv)].astype(np.float64) @ q[b, h].astype(np.float16).astype(np.float64) * SCALE
+            p = np.exp(s - s.max())
+            ref = p @ vc[:n, h // (n_q // n_kv)].astype(np.float64) / p.sum()
+            assert rel_l2(got[b, h], ref) <= TOL, (b, h)

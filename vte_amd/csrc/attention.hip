@@ -23,10 +23,12 @@
 //    blocks past a sequence's last split exit at once, and the combine reads
 //    only that sequence's splits, so each sequence's result is independent of
 //    the batch it sits in.
+#include <algorithm>
 #include <cstdlib>
 #include "vte_common.h"
 
 #include "attn_tile.h"
+#include "attn_prompt.h"
 
 
 // ---------------------------------------------------------------------------
@@ -477,10 +479,41 @@ static bool getenv_off_att(const char* name) {
     return v != nullptr && atoi(v) == 0;
 }
 
+// Many columns of one cache (a prompt chunk's): rows of 64 instead of pairs of
+// columns per K/V read.  512 columns after 1536 rows 77.5 -> 21.8 us (start 0:
+// 28.1 -> 13.3), 128 columns 23.8 -> 13.2, 80 columns 18.9 -> 12.8; at 64 columns
+// and fewer the two-column blocks, which give the bits of the decode path.
+static bool prompt_form(int B, int n_q, int kv_batch_stride, int split, float scale, const void* out,
+                        const int* counters) {
+    return kv_batch_stride == 0 && B > 64 && counters == nullptr && out != nullptr && scale > 0.f &&
+           !getenv_off_att("VTE_ATT_QC");
+}
+
+template <typename TQ, typename TO>
+static hipError_t attn_prompt(const void* q, const void* k_cache, const void* v_cache, float* part_m, float* part_l,
+                              float* part_o, void* out, int B, int n_q, int n_kv, float scale, const int* kv_offset,
+                              int max_ctx, int max_splits, hipStream_t st) {
+    // token shares: as many as two blocks per CU hold (512 columns of 12 heads,
+    // 2048 rows: 256 / 512 / 768 blocks 30.5 / 23.0 / 25.9 us), of 128 rows at least
+    const int rbs = (B * (n_q / n_kv) + AP_ROWS - 1) / AP_ROWS;
+    const int nsp = std::max(1, std::min({AP_MAX_SPLITS, max_splits, max_ctx / 128, 512 / (rbs * n_kv)}));
+    hipLaunchKernelGGL((attn_prompt_kernel<TQ, TO>), dim3(rbs, n_kv, nsp), dim3(256), 0, st, (const TQ*)q,
+                       (const __half*)k_cache, (const __half*)v_cache, part_m, part_l, part_o, (TO*)out, n_q, n_kv,
+                       scale, kv_offset, B, max_ctx, max_splits);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || nsp == 1) return e;
+    hipLaunchKernelGGL((attn_prompt_combine<TO>), dim3((B * n_q + 7) / 8), dim3(256), 0, st, part_m, part_l, part_o,
+                       (TO*)out, B * n_q, nsp, max_splits);
+    return hipGetLastError();
+}
+
 template <typename TQ, typename TO>
 hipError_t attn_split_kv(const void* q, const void* k_cache, const void* v_cache, float* part_m, float* part_l,
                          float* part_o, void* out, int B, int n_q, int n_kv, float scale, const int* kv_offset,
                          int kv_batch_stride, int split, int max_splits, int* counters, hipStream_t st) {
+    if (prompt_form(B, n_q, kv_batch_stride, split, scale, out, counters))
+        return attn_prompt<TQ, TO>(q, k_cache, v_cache, part_m, part_l, part_o, out, B, n_q, n_kv, scale, kv_offset,
+                                   (int)std::min(2147483647LL, (long long)max_splits * split), max_splits, st);
     dim3 g1(max_splits, n_kv, B), b1(256);
     // positions every split may read ahead of knowing the length: all of
     // max_splits * split must lie inside one sequence's kv_batch_stride
