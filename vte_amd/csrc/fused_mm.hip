@@ -111,10 +111,9 @@ __device__ __forceinline__ const uint8_t* mm_row(const MmTile& T, int rr) {
 }
 
 template <int FMT, int RT, int NT, int NW>
-__device__ __forceinline__ void mm_body(const MmPlan& P, const MmTile& T, float (*red)[RT][NT][4][64],
-                                        float (*xl)[NT * 128]) {
+__device__ __forceinline__ void mm_body(const MmPlan& P, const MmTile& T, MfWave<RT, NT, NT == 1>* L) {
     constexpr bool XM = NT > 1;  // minimum-term form (q4_xmin)
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, grp = lane >> 4;
     const int K = P.K, M = P.M, n_sb = K / QK_K;
     const int sb0 = (n_sb * wv) / NW, sb1 = (n_sb * (wv + 1)) / NW;
@@ -130,6 +129,16 @@ __device__ __forceinline__ void mm_body(const MmPlan& P, const MmTile& T, float 
     for (int rt = 0; rt < RT; ++rt) rowp[rt] = mm_row<RT>(T, rt * 16 + col);
 
     for (int sb = sb0; sb < sb1; ++sb) {
+        if constexpr (NT == 1) {  // staged activations: no registers in flight, so more blocks per CU
+            sb_stage_x(x, K, sb, M, L[wv].x, lane);
+            typename SbRaw<FMT>::Raw raw[RT];
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+                sb_load(rowp[rt] + (size_t)sb * (FMT == 4 ? Q4K_BYTES : Q6K_BYTES), grp, raw[rt]);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            sb_staged<RT>(raw, L[wv].x, col, grp, acc);
+            continue;
+        } else {
         half8_t bx[8][NT];
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
@@ -147,12 +156,13 @@ __device__ __forceinline__ void mm_body(const MmPlan& P, const MmTile& T, float 
         for (int rt = 0; rt < RT; ++rt)
             sb_load(rowp[rt] + (size_t)sb * (FMT == 4 ? Q4K_BYTES : Q6K_BYTES), grp, raw[rt]);
         XMin<NT, XM> xm;
-        sb_xmin<FMT, NT, XM>(bx, xl[wv], xm);
+        sb_xmin<FMT, NT, XM>(bx, L[wv].xl, xm);
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
             typename SbRaw<FMT>::Ops ops;
             sb_ops<XM>(raw[rt], grp, ops);
             sb_mfma<NT>(ops, bx, xm, acc[rt]);
+        }
         }
     }
 #pragma unroll
@@ -160,18 +170,18 @@ __device__ __forceinline__ void mm_body(const MmPlan& P, const MmTile& T, float 
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) red[wv][rt][nt][i][lane] = acc[rt][nt][i];
+            for (int i = 0; i < 4; ++i) L[wv].red[rt][nt][i][lane] = acc[rt][nt][i];
 }
 
 // Sum over the NW waves of tile row rr, batch column mc (C layout: lane
 // (row rw, grp) holds batch columns 4*grp+i of a 16-column tile).
-template <int RT, int NT, int NW>
-__device__ __forceinline__ float mm_sum(float (*red)[RT][NT][4][64], int rr, int mc) {
+template <int RT, int NT, int NW, bool ST>
+__device__ __forceinline__ float mm_sum(const MfWave<RT, NT, ST>* L, int rr, int mc) {
     const int rt = rr >> 4, rw = rr & 15, nt = mc >> 4, cc = mc & 15;
     const int ln = c_lane(rw, cc), i = c_reg(cc);
     float s = 0.f;
 #pragma unroll
-    for (int wq = 0; wq < NW; ++wq) s += red[wq][rt][nt][i][ln];
+    for (int wq = 0; wq < NW; ++wq) s += L[wq].red[rt][nt][i][ln];
     return s;
 }
 
@@ -212,37 +222,36 @@ __device__ __forceinline__ void mm_put_pair(const MmPlan& P, const MmSeg& S, int
 }
 
 // Epilogue of a block's C tiles: batch columns cb .. cb + mcount - 1.
-template <int RT, int NT, int NW>
-__device__ __forceinline__ void mm_epilogue(const MmPlan& P, const MmTile& T, float (*red)[RT][NT][4][64], int cb,
+template <int RT, int NT, int NW, bool ST>
+__device__ __forceinline__ void mm_epilogue(const MmPlan& P, const MmTile& T, const MfWave<RT, NT, ST>* L, int cb,
                                             int mcount) {
     const MmSeg& S = *T.S;
     if (!mm_paired(S.mode)) {
         for (int o = threadIdx.x; o < 16 * RT * 16 * NT; o += blockDim.x) {
             const int rr = o / (16 * NT), mc = o % (16 * NT);
-            if (rr < T.nvalid && mc < mcount) mm_put(P, S, T.j0 + rr, cb + mc, mm_sum<RT, NT, NW>(red, rr, mc));
+            if (rr < T.nvalid && mc < mcount) mm_put(P, S, T.j0 + rr, cb + mc, mm_sum<RT, NT, NW>(L, rr, mc));
         }
         return;
     }
     for (int o = threadIdx.x; o < 8 * RT * 16 * NT; o += blockDim.x) {
         const int p = o / (16 * NT), mc = o % (16 * NT);
         if (p < T.nvalid && mc < mcount)
-            mm_put_pair(P, S, T.j0 + p, cb + mc, mm_sum<RT, NT, NW>(red, p, mc),
-                        mm_sum<RT, NT, NW>(red, p + 8 * RT, mc));
+            mm_put_pair(P, S, T.j0 + p, cb + mc, mm_sum<RT, NT, NW>(L, p, mc),
+                        mm_sum<RT, NT, NW>(L, p + 8 * RT, mc));
     }
 }
 
 // NW waves per block split K (6 for K = 1536: one super-block each).
-template <int RT, int NT, int NW>
-__global__ __launch_bounds__(64 * NW, RT == 2 && NT == 1 ? 4 : 1) void fused_mm_kernel(MmPlan P) {
-    __shared__ float red[NW][RT][NT][4][64];
-    __shared__ float xl[NW][NT * 128];  // minimum-term scratch per wave (q4_xmin)
+template <int RT, int NT, int NW, bool Q6>
+__global__ __launch_bounds__(64 * NW, RT == 2 && NT == 1 && NW == 6 ? 5 : 1) void fused_mm_kernel(MmPlan P) {
+    __shared__ MfWave<RT, NT, NT == 1> L[NW];
     const MmTile T = mm_tile<RT>(P, blockIdx.x);
     const MmSeg& S = *T.S;
-    if (S.fmt == 4) mm_body<4, RT, NT, NW>(P, T, red, xl);
-    else mm_body<6, RT, NT, NW>(P, T, red, xl);
+    if (!Q6 || S.fmt == 4) mm_body<4, RT, NT, NW>(P, T, L);
+    else mm_body<6, RT, NT, NW>(P, T, L);
     __syncthreads();
 
-    mm_epilogue<RT, NT, NW>(P, T, red, 0, P.M);
+    mm_epilogue<RT, NT, NW>(P, T, L, 0, P.M);
 }
 
 
@@ -255,8 +264,7 @@ __global__ __launch_bounds__(64 * NW, RT == 2 && NT == 1 ? 4 : 1) void fused_mm_
 // its eight k-steps in the same order as fused_mm_kernel, so both forms give
 // the same bits.
 template <int FMT, int RT, int NT>
-__device__ __forceinline__ void mm_ws_body(const MmPlan& P, const MmTile& T, float (*red)[RT][NT][4][64],
-                                           float (*xl)[NT * 128], int c0,
+__device__ __forceinline__ void mm_ws_body(const MmPlan& P, const MmTile& T, MfWave<RT, NT, false>* L, int c0,
                                            int c1) {
     constexpr bool XM = true;  // minimum-term form (q4_xmin)
     constexpr int NW = 6;
@@ -291,7 +299,7 @@ __device__ __forceinline__ void mm_ws_body(const MmPlan& P, const MmTile& T, flo
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) acc[rt][nt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
         XMin<NT, XM> xm;
-        sb_xmin<FMT, NT, XM>(bx, xl[wv], xm);
+        sb_xmin<FMT, NT, XM>(bx, L[wv].xl, xm);
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) sb_mfma<NT>(ops[rt], bx, xm, acc[rt]);
 #pragma unroll
@@ -299,23 +307,22 @@ __device__ __forceinline__ void mm_ws_body(const MmPlan& P, const MmTile& T, flo
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) red[wv][rt][nt][i][lane] = acc[rt][nt][i];
+                for (int i = 0; i < 4; ++i) L[wv].red[rt][nt][i][lane] = acc[rt][nt][i];
         if (m0 + 16 * NT < c1) load_b(m0 + 16 * NT);
         __syncthreads();
-        mm_epilogue<RT, NT, NW>(P, T, red, m0, min(16 * NT, c1 - m0));
+        mm_epilogue<RT, NT, NW>(P, T, L, m0, min(16 * NT, c1 - m0));
         __syncthreads();
     }
 }
 
 template <int RT, int NT>
 __global__ __launch_bounds__(64 * 6) void fused_mm_ws_kernel(MmPlan P, int cols) {
-    __shared__ float red[6][RT][NT][4][64];
-    __shared__ float xl[6][NT * 128];
+    __shared__ MfWave<RT, NT, false> L[6];
     const MmTile T = mm_tile<RT>(P, blockIdx.x);
     const int c0 = blockIdx.y * cols, c1 = min(P.M, c0 + cols);
     if (c0 >= c1) return;
-    if (T.S->fmt == 4) mm_ws_body<4, RT, NT>(P, T, red, xl, c0, c1);
-    else mm_ws_body<6, RT, NT>(P, T, red, xl, c0, c1);
+    if (T.S->fmt == 4) mm_ws_body<4, RT, NT>(P, T, L, c0, c1);
+    else mm_ws_body<6, RT, NT>(P, T, L, c0, c1);
 }
 
 // Eight SwiGLU outputs of column m from the sums of eight gate and up rows.
@@ -468,6 +475,8 @@ static hipError_t mm_run(MmPlan P, int B, MmForm form, size_t out_ld_elems[MM_MA
     for (int s = 0; s < P.nseg; ++s) out0[s] = P.seg[s].out;
     __half* kc0 = P.k_cache;
     __half* vc0 = P.v_cache;
+    bool q6 = false;
+    for (int s = 0; s < P.nseg; ++s) q6 = q6 || P.seg[s].fmt != 4;
     if constexpr (RT == 4) if (form == MM_WS) {
         // 64 rows per block, 16 columns at a time: one block per CU
         const int g = ws_column_groups(total, B, device_cus());
@@ -495,13 +504,22 @@ static hipError_t mm_run(MmPlan P, int B, MmForm form, size_t out_ld_elems[MM_MA
         // batches above 16 columns take the two-tile form for every chunk, a
         // short tail included, so all their columns share the minimum-term
         // form (and the bits) of the weight-stationary launch
+#define MM_LAUNCH(NT_, NW_, Q6_) \
+    hipLaunchKernelGGL((fused_mm_kernel<RT, NT_, NW_, Q6_>), dim3(total), dim3(64 * NW_), 0, st, P)
+#define MM_LAUNCH_Q(NT_, NW_)                    \
+    do {                                         \
+        if (q6) MM_LAUNCH(NT_, NW_, true);       \
+        else MM_LAUNCH(NT_, NW_, false);         \
+    } while (0)
         if (P.K == 6 * QK_K) {
-            if (B > 16) hipLaunchKernelGGL((fused_mm_kernel<RT, 2, 6>), dim3(total), dim3(64 * 6), 0, st, P);
-            else hipLaunchKernelGGL((fused_mm_kernel<RT, 1, 6>), dim3(total), dim3(64 * 6), 0, st, P);
+            if (B > 16) MM_LAUNCH_Q(2, 6);
+            else MM_LAUNCH_Q(1, 6);
         } else {
-            if (B > 16) hipLaunchKernelGGL((fused_mm_kernel<RT, 2, MF_WAVES>), dim3(total), dim3(64 * MF_WAVES), 0, st, P);
-            else hipLaunchKernelGGL((fused_mm_kernel<RT, 1, MF_WAVES>), dim3(total), dim3(64 * MF_WAVES), 0, st, P);
+            if (B > 16) MM_LAUNCH_Q(2, MF_WAVES);
+            else MM_LAUNCH_Q(1, MF_WAVES);
         }
+#undef MM_LAUNCH_Q
+#undef MM_LAUNCH
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }

@@ -27,11 +27,10 @@ template <typename TI, typename TO, int FMT, int RT, int NT, int NW>
 __device__ __forceinline__ void gemm_mfma_body(const TI* __restrict__ x, const uint8_t* __restrict__ w,
                                                TO* __restrict__ y, int M, int K, int N, const TO* __restrict__ bias,
                                                const TO* __restrict__ residual, float rs, size_t split_stride,
-                                               int split, int nsplit, float (*red)[RT][NT][4][64],
-                                               float (*xl)[NT * 128]) {
+                                               int split, int nsplit, MfWave<RT, NT, NT == 1>* L) {
     constexpr bool XM = NT > 1;  // minimum-term form (q4_xmin)
 
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, grp = lane >> 4;
     const int n_sb = K / QK_K;
     const int bpr = (FMT == 4) ? Q4K_BYTES : Q6K_BYTES;
@@ -50,6 +49,16 @@ __device__ __forceinline__ void gemm_mfma_body(const TI* __restrict__ x, const u
         for (int nt = 0; nt < NT; ++nt) acc[rt][nt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
 
     for (int sb = sb0; sb < sb1; ++sb) {
+        if constexpr (NT == 1) {  // staged activations: coalesced, and fp16 holds no registers in flight
+            sb_stage_x(x, K, sb, M, L[wv].x, lane);
+            typename SbRaw<FMT>::Raw raw[RT];
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+                sb_load(w + (size_t)min(row0 + rt * 16 + col, N - 1) * row_bytes + (size_t)sb * bpr, grp, raw[rt]);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            sb_staged<RT>(raw, L[wv].x, col, grp, acc);
+            continue;
+        } else {
         // ---- A operands (activations) for the 8 k-steps ----
         half8_t bx[8][NT];
 #pragma unroll
@@ -70,12 +79,13 @@ __device__ __forceinline__ void gemm_mfma_body(const TI* __restrict__ x, const u
             sb_load(w + (size_t)r * row_bytes + (size_t)sb * bpr, grp, raw[rt]);
         }
         XMin<NT, XM> xm;
-        sb_xmin<FMT, NT, XM>(bx, xl[wv], xm);
+        sb_xmin<FMT, NT, XM>(bx, L[wv].xl, xm);
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
             typename SbRaw<FMT>::Ops ops;
             sb_ops<XM>(raw[rt], grp, ops);
             sb_mfma<NT>(ops, bx, xm, acc[rt]);
+        }
         }
     }
 
@@ -85,7 +95,7 @@ __device__ __forceinline__ void gemm_mfma_body(const TI* __restrict__ x, const u
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) red[wv][rt][nt][i][lane] = acc[rt][nt][i];
+            for (int i = 0; i < 4; ++i) L[wv].red[rt][nt][i][lane] = acc[rt][nt][i];
     __syncthreads();
     // C layout: lane (row rw, grp) holds batch columns 4*grp + i of the tile.
     for (int o = threadIdx.x; o < RT * 16 * NT * 16; o += blockDim.x) {
@@ -94,7 +104,7 @@ __device__ __forceinline__ void gemm_mfma_body(const TI* __restrict__ x, const u
         const int ln = c_lane(rw, cc), i = c_reg(cc);
         float s = 0.f;
 #pragma unroll
-        for (int wq = 0; wq < NW; ++wq) s += red[wq][rt][nt][i][ln];
+        for (int wq = 0; wq < NW; ++wq) s += L[wq].red[rt][nt][i][ln];
         const int row = row0 + rr;
         if (row < N && mc < M) gemv_store<TO>(y, bias, residual, rs, row, mc, N, s);
     }
@@ -106,10 +116,9 @@ __global__ __launch_bounds__(64 * NW, RT == 2 && NT == 1 ? 4 : 1) void gemm_mfma
                                                         TO* __restrict__ y, int M, int K, int N,
                                                         const TO* __restrict__ bias, const TO* __restrict__ residual,
                                                         float rs, size_t split_stride) {
-    __shared__ float red[NW][RT][NT][4][64];
-    __shared__ float xl[NW][NT * 128];  // minimum-term scratch per wave (q4_xmin)
+    __shared__ MfWave<RT, NT, NT == 1> L[NW];
     gemm_mfma_body<TI, TO, FMT, RT, NT, NW>(x, w, y, M, K, N, bias, residual, rs, split_stride, (int)blockIdx.y,
-                                            (int)gridDim.y, red, xl);
+                                            (int)gridDim.y, L);
 }
 
 // Batched MFMA GEMM behind the reference GEMV's 10-argument ABI (fp16 I/O,
@@ -122,8 +131,7 @@ template <int FMT>
 __device__ __forceinline__ void gemm_ref_abi(const void* input_ptr, const void* weight_ptr, void* output_ptr, int batch,
                                              int seq_len, int in_features, int out_features, const void* bias_ptr,
                                              const void* residual_ptr, float residual_scale) {
-    __shared__ float red[MF_WAVES][2][1][4][64];
-    __shared__ float xl[MF_WAVES][128];
+    __shared__ MfWave<2, 1, true> L[MF_WAVES];
     const int cols = batch * seq_len, c0 = (int)blockIdx.y * 16;
     if (c0 >= cols) return;
     const __half* x = static_cast<const __half*>(input_ptr) + (size_t)c0 * in_features;
@@ -132,7 +140,7 @@ __device__ __forceinline__ void gemm_ref_abi(const void* input_ptr, const void* 
     gemm_mfma_body<__half, __half, FMT, 2, 1, MF_WAVES>(x, static_cast<const uint8_t*>(weight_ptr), y,
                                                         min(16, cols - c0), in_features, out_features,
                                                         static_cast<const __half*>(bias_ptr), res, residual_scale, 0,
-                                                        0, 1, red, xl);
+                                                        0, 1, L);
 }
 extern "C" __global__ __launch_bounds__(64 * MF_WAVES) void gemm_q4k_mfma_kernel(
     const void* input_ptr, const void* weight_ptr, void* output_ptr, int batch, int seq_len, int in_features,

@@ -376,6 +376,103 @@ __device__ __forceinline__ void sb_ops(const Q4Raw& r, int grp, Q4Ops& o) { q4_e
 template <bool XM>
 __device__ __forceinline__ void sb_ops(const Q6Raw& r, int grp, Q6Ops& o) { q6_exact_operands(r, grp, o); }
 
+// LDS of one wave of a batched kernel: its partial C tiles, summed over the
+// waves by the epilogue, over its staged activations (ST, 16 columns), and the
+// minimum-term scratch (q4_xmin).
+template <int RT, int NT, bool ST>
+struct alignas(16) MfWave {
+    union {
+        _Float16 x[ST ? 16 * QK_K : 8];
+        float red[RT][NT][4][64];
+    };
+    float xl[ST ? 4 : NT * 128];
+};
+
+// 16 columns' activations of super-block sb into a wave's LDS as fp16 rows of
+// 256, 16-byte chunks permuted by chunk ^ column so an operand read's 16
+// columns lie in distinct banks; columns past M stay as they are (results
+// unused).  Consecutive lanes take consecutive bytes, and fp16 goes straight
+// to LDS, holding no registers (wait for vmcnt before reading it).
+__device__ __forceinline__ void sb_stage_x(const __half* x, int K, int sb, int M, _Float16* lds, int lane) {
+    asm volatile("" : "+v"(lane));  // addresses made here, not kept across the loop over super-blocks
+    const int hi = lane >> 5, slot = lane & 31;
+    const char* base = reinterpret_cast<const char*>(x + sb * QK_K);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        if (2 * j >= M) break;
+        const uint32_t off = 2u * (uint32_t)(min(2 * j + hi, M - 1) * K) + 16u * (uint32_t)(slot ^ (2 * j + hi));
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(base + off),
+                                         (__attribute__((address_space(3))) void*)(lds + 2 * j * QK_K), 16, 0, 0);
+    }
+}
+__device__ __forceinline__ void sb_stage_x(const float* x, int K, int sb, int M, _Float16* lds, int lane) {
+    typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+    float4 v[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j)  // (a repeated row costs less than the branches that would skip it)
+        v[j] = reinterpret_cast<const float4*>(x + (size_t)min(j, M - 1) * K + sb * QK_K)[lane];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        const int slot = (lane >> 1) ^ j;
+        *reinterpret_cast<half4_t*>(lds + j * QK_K + 8 * slot + 4 * (lane & 1)) =
+            half4_t{(_Float16)v[j].x, (_Float16)v[j].y, (_Float16)v[j].z, (_Float16)v[j].w};
+    }
+}
+
+// One super-block of sb_mfma's work (minimum term per k-step) for RT row tiles
+// and 16 staged columns, each k-step's operands made as they are needed.
+template <int RT>
+__device__ __forceinline__ void sb_staged(const Q4Raw (&r)[RT], const _Float16* x, int col, int grp,
+                                          floatx4_t (&acc)[RT][1]) {
+    floatx4_t aw[RT], am[RT];
+    uint32_t sc[RT][2], mn[RT][2];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        aw[rt] = am[rt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+        q4_scale_words(r[rt].h, sc[rt]);
+        q4_min_words(r[rt].h, mn[rt]);
+    }
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        const int ci = t >> 2, part = (t >> 1) & 1, b = 2 * (grp >> 1) + part;
+        const half8_t xv = *reinterpret_cast<const half8_t*>(x + col * QK_K + 8 * ((kslot_base<4>(t, grp) >> 3) ^ col));
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            const half2_t s2 = byte_splat(sc[rt][ci], b), m = byte_splat(mn[rt][ci], b);
+            const half8_t wv = q4_step_operand(ci == 0 ? r[rt].q0 : r[rt].q1, part, t & 1, s2, s2 * splat2(-1024.0f));
+            const half8_t mv = {m[0], m[1], m[0], m[1], m[0], m[1], m[0], m[1]};
+            aw[rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv, wv, aw[rt], 0, 0, 0);
+            am[rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv, mv, am[rt], 0, 0, 0);
+        }
+        if (t & 1) __builtin_amdgcn_sched_barrier(0);  // two steps' operands at a time, not all eight
+    }
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        const float d = h2f_bits(r[rt].h.x), dmin = h2f_bits(r[rt].h.x >> 16);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[rt][0][i] = fmaf(-dmin, am[rt][i], fmaf(d, aw[rt][i], acc[rt][0][i]));
+    }
+}
+template <int RT>
+__device__ __forceinline__ void sb_staged(const Q6Raw (&r)[RT], const _Float16* x, int col, int grp,
+                                          floatx4_t (&acc)[RT][1]) {
+    floatx4_t aw[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) aw[rt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        const half8_t xv = *reinterpret_cast<const half8_t*>(x + col * QK_K + 8 * ((kslot_base<6>(t, grp) >> 3) ^ col));
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+            aw[rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv, q6_step_operand(r[rt], t, grp), aw[rt], 0, 0, 0);
+        if (t & 1) __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[rt][0][i] = fmaf(h2f_bits(r[rt].d), aw[rt][i], acc[rt][0][i]);
+}
+
 // C tile element of weight row rw (0..15) and batch column cc (0..15): lane
 // rw + 16 * (cc / 4), register cc % 4.
 __device__ __forceinline__ int c_lane(int rw, int cc) { return rw + 16 * (cc >> 2); }
