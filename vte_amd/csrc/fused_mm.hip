@@ -222,19 +222,21 @@ __device__ __forceinline__ void mm_put_pair(const MmPlan& P, const MmSeg& S, int
 }
 
 // Epilogue of a block's C tiles: batch columns cb .. cb + mcount - 1.
+// Neighbouring lanes take neighbouring rows: contiguous stores, and LDS reads
+// of distinct banks.
 template <int RT, int NT, int NW, bool ST>
 __device__ __forceinline__ void mm_epilogue(const MmPlan& P, const MmTile& T, const MfWave<RT, NT, ST>* L, int cb,
                                             int mcount) {
     const MmSeg& S = *T.S;
     if (!mm_paired(S.mode)) {
         for (int o = threadIdx.x; o < 16 * RT * 16 * NT; o += blockDim.x) {
-            const int rr = o / (16 * NT), mc = o % (16 * NT);
+            const int rr = o % (16 * RT), mc = o / (16 * RT);
             if (rr < T.nvalid && mc < mcount) mm_put(P, S, T.j0 + rr, cb + mc, mm_sum<RT, NT, NW>(L, rr, mc));
         }
         return;
     }
     for (int o = threadIdx.x; o < 8 * RT * 16 * NT; o += blockDim.x) {
-        const int p = o / (16 * NT), mc = o % (16 * NT);
+        const int p = o % (8 * RT), mc = o / (8 * RT);
         if (p < T.nvalid && mc < mcount)
             mm_put_pair(P, S, T.j0 + p, cb + mc, mm_sum<RT, NT, NW>(L, p, mc),
                         mm_sum<RT, NT, NW>(L, p + 8 * RT, mc));

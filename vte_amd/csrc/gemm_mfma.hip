@@ -99,7 +99,7 @@ __device__ __forceinline__ void gemm_mfma_body(const TI* __restrict__ x, const u
     __syncthreads();
     // C layout: lane (row rw, grp) holds batch columns 4*grp + i of the tile.
     for (int o = threadIdx.x; o < RT * 16 * NT * 16; o += blockDim.x) {
-        const int rr = o / (NT * 16), mc = o % (NT * 16);
+        const int rr = o % (RT * 16), mc = o / (RT * 16);
         const int rt = rr >> 4, rw = rr & 15, nt = mc >> 4, cc = mc & 15;
         const int ln = c_lane(rw, cc), i = c_reg(cc);
         float s = 0.f;
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(64 * MF_WAVES) void gemm_ws_splitk_kernel(const __h
         __syncthreads();
         const int mcount = min(16 * NT, c1 - m0);
         for (int o = threadIdx.x; o < 16 * RT * NT * 16; o += blockDim.x) {
-            const int rr = o / (NT * 16), mc = o % (NT * 16);
+            const int rr = o % (RT * 16), mc = o / (RT * 16);
             const int rt = rr >> 4, rw = rr & 15, nt = mc >> 4, cc = mc & 15;
             const int ln = c_lane(rw, cc), i = c_reg(cc);
             float s = 0.f;
