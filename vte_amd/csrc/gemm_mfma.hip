@@ -163,16 +163,17 @@ extern "C" __global__ __launch_bounds__(64 * MF_WAVES) void gemm_q6k_mfma_kernel
 // columns [blockIdx.z * cols, ...), 16 * NT at a time, requesting the next
 // columns' activations before the epilogue; the k-steps and the wave sum keep
 // the order of gemm_mfma_kernel, so the partial sums have the same bits.
-template <int FMT, int RT, int NT>
+template <int FMT, int RT>
 __global__ __launch_bounds__(64 * MF_WAVES) void gemm_ws_splitk_kernel(const __half* __restrict__ x,
                                                                      const uint8_t* __restrict__ w,
                                                                      float* __restrict__ part, int M, int K, int N,
                                                                      size_t split_stride, int cols) {
     constexpr bool XM = true;  // minimum-term form (q4_xmin)
-    constexpr int NW = MF_WAVES;
+    constexpr int NW = MF_WAVES, NT = 1;
+    __shared__ alignas(16) _Float16 xb[NW][16 * QK_K];
     __shared__ float red[NW][RT][NT][4][64];
     __shared__ float xl[NW][NT * 128];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, grp = lane >> 4;
     const int n_sb = K / QK_K;
     const size_t row_bytes = (size_t)n_sb * (FMT == 4 ? Q4K_BYTES : Q6K_BYTES);
@@ -194,17 +195,8 @@ __global__ __launch_bounds__(64 * MF_WAVES) void gemm_ws_splitk_kernel(const __h
             sb_ops<XM>(raw, grp, ops[rt]);
         }
     }
-    half8_t bx[8][NT];
     auto load_b = [&](int m0) {
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const int kb = sb0 * QK_K + kslot_base<FMT>(t, grp);
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                const int m = m0 + nt * 16 + col;
-                bx[t][nt] = load_x8<__half>(x + (size_t)(m < c1 ? m : c0) * K + kb, has && m < c1);
-            }
-        }
+        if (has) sb_stage_x(x + (size_t)m0 * K, K, sb0, c1 - m0, xb[wv], lane);
     };
     load_b(c0);
     for (int m0 = c0; m0 < c1; m0 += 16 * NT) {
@@ -214,6 +206,11 @@ __global__ __launch_bounds__(64 * MF_WAVES) void gemm_ws_splitk_kernel(const __h
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) acc[rt][nt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
         if (has) {
+            half8_t bx[8][NT];
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's copies; no other wave reads them
+            sb_read_x<FMT>(xb[wv], col, grp, bx);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read: the next columns may land
+            if (m0 + 16 < c1) load_b(m0 + 16);
             XMin<NT, XM> xm;
             sb_xmin<FMT, NT, XM>(bx, xl[wv], xm);
 #pragma unroll
@@ -225,7 +222,6 @@ __global__ __launch_bounds__(64 * MF_WAVES) void gemm_ws_splitk_kernel(const __h
             for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) red[wv][rt][nt][i][lane] = acc[rt][nt][i];
-        if (m0 + 16 * NT < c1) load_b(m0 + 16 * NT);
         __syncthreads();
         const int mcount = min(16 * NT, c1 - m0);
         for (int o = threadIdx.x; o < 16 * RT * NT * 16; o += blockDim.x) {
@@ -559,7 +555,7 @@ static hipError_t launch_splitk(const void* x, const void* w, float* part, int M
         const int tiles = (N + 63) / 64;
         const int g = ws_column_groups(tiles * splits, M, device_cus());
         const int cols = ((M + 31) / 32 + g - 1) / g * 32, gz = (M + cols - 1) / cols;
-        hipLaunchKernelGGL((gemm_ws_splitk_kernel<FMT, 4, 1>), dim3(tiles, splits, gz), dim3(64 * MF_WAVES), 0, st,
+        hipLaunchKernelGGL((gemm_ws_splitk_kernel<FMT, 4>), dim3(tiles, splits, gz), dim3(64 * MF_WAVES), 0, st,
                            (const __half*)x, (const uint8_t*)w, part, M, K, N, ss, cols);
         return hipGetLastError();
     }

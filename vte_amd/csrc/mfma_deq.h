@@ -419,6 +419,14 @@ __device__ __forceinline__ void sb_stage_x(const float* x, int K, int sb, int M,
     }
 }
 
+// The eight operands of a staged column tile.
+template <int FMT, int NT>
+__device__ __forceinline__ void sb_read_x(const _Float16* x, int col, int grp, half8_t (&bx)[8][NT]) {
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+        bx[t][0] = *reinterpret_cast<const half8_t*>(x + col * QK_K + 8 * ((kslot_base<FMT>(t, grp) >> 3) ^ col));
+}
+
 // One super-block of sb_mfma's work (minimum term per k-step) for RT row tiles
 // and 16 staged columns, each k-step's operands made as they are needed.
 template <int RT>

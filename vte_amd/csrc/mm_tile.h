@@ -240,9 +240,10 @@ __device__ __forceinline__ void mt_loop(const TI* __restrict__ x, int K, int c0,
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
         }
-        // Products, half a super-block (four k-steps) at a time: the next half's
-        // operands are requested from LDS ahead of this half's MFMAs.  The scheduling barriers keep
-        // the compiler from requesting more ahead than the registers hold.
+        // Products, half a super-block (four k-steps) at a time: under this half's
+        // MFMAs the next half's operands are requested from LDS and a row tile of
+        // the column tile before is scaled (an MFMA leaves two issue slots free
+        // while it runs; the group barriers put the other instructions there).
         half8_t b0[4], b1[4], xa = {0, 0, 0, 0, 0, 0, 0, 0};
         auto fetch = [&](half8_t (&b)[4], int nt, int h) {
 #pragma unroll
@@ -252,13 +253,23 @@ __device__ __forceinline__ void mt_loop(const TI* __restrict__ x, int K, int c0,
         auto fetch_xs = [&](int nt) {  // groups 2, 3 read them too: their minima are zero
             if constexpr (FMT == 4) xa = *reinterpret_cast<const half8_t*>(L.xs + (nt * 16 + col) * 16 + 8 * (grp & 1));
         };
-        floatx4_t aw[2], am[2];
+        auto interleave = [] {
+#pragma unroll
+            for (int i = 0; i < 10; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
+                __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // VALU
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        __builtin_amdgcn_s_setprio(1);
+        floatx4_t aw[2], am[2], pw[2], pm[2];
         fetch_xs(0);
         fetch(b0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
             fetch(b1, nt, 1);
-            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int rt = 0; rt < 2; ++rt) {
                 aw[rt] = am[rt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
@@ -269,21 +280,28 @@ __device__ __forceinline__ void mt_loop(const TI* __restrict__ x, int K, int c0,
 #pragma unroll
                 for (int rt = 0; rt < 2; ++rt)
                     aw[rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b0[t], ops[rt].w[t], aw[rt], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
+            if (nt > 0) mt_add(ops[0], pw[0], pm[0], acc[0][nt - 1]);
+            interleave();
             if (nt + 1 < NT) {
                 fetch_xs(nt + 1);
                 fetch(b0, nt + 1, 0);
             }
-            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int t = 0; t < 4; ++t)
 #pragma unroll
                 for (int rt = 0; rt < 2; ++rt)
                     aw[rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b1[t], ops[rt].w[4 + t], aw[rt], 0, 0, 0);
+            if (nt > 0) mt_add(ops[1], pw[1], pm[1], acc[1][nt - 1]);
+            interleave();
 #pragma unroll
-            for (int rt = 0; rt < 2; ++rt) mt_add(ops[rt], aw[rt], am[rt], acc[rt][nt]);
-            __builtin_amdgcn_sched_barrier(0);
+            for (int rt = 0; rt < 2; ++rt) {
+                pw[rt] = aw[rt];
+                pm[rt] = am[rt];
+            }
         }
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) mt_add(ops[rt], pw[rt], pm[rt], acc[rt][NT - 1]);
+        __builtin_amdgcn_s_setprio(0);
         // the products are done with this super-block's LDS
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
         __builtin_amdgcn_s_barrier();
