@@ -266,15 +266,15 @@ __global__ __launch_bounds__(64 * NW, RT == 2 && NT == 1 && NW == 6 ? 5 : 1) voi
 // super-blocks:
 // wave w decodes super-block w of its tile rows once, keeps the weight
 // operands in registers and runs them against the block's columns
-// [blockIdx.y * cols, ...) 16 * NT at a time, the next columns' activations
+// [blockIdx.y * cols, ...) 16 at a time, the next columns' activations
 // requested ahead.  Each C tile sums
 // its eight k-steps in the same order as fused_mm_kernel, so both forms give
 // the same bits.
-template <int FMT, int RT, int NT>
-__device__ __forceinline__ void mm_ws_body(const MmPlan& P, const MmTile& T, MfWave<RT, NT, false>* L,
+template <int FMT, int RT>
+__device__ __forceinline__ void mm_ws_body(const MmPlan& P, const MmTile& T, MfWave<RT, 1, false>* L,
                                            _Float16 (*xb)[16 * QK_K], int c0, int c1) {
     constexpr bool XM = true;  // minimum-term form (q4_xmin)
-    constexpr int NW = 6;
+    constexpr int NW = 6, NT = 1;
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, grp = lane >> 4;
     const int K = P.K;
@@ -286,24 +286,7 @@ __device__ __forceinline__ void mm_ws_body(const MmPlan& P, const MmTile& T, MfW
         sb_load(rowp + (size_t)wv * (FMT == 4 ? Q4K_BYTES : Q6K_BYTES), grp, raw);
         sb_ops<XM>(raw, grp, ops[rt]);
     }
-    // Activations of the columns from m0: one 16-column tile is staged in the
-    // wave's LDS, two tiles go to registers.
-    half8_t bx[8][NT];
-    auto load_b = [&](int m0) {
-        if constexpr (NT == 1) {
-            sb_stage_x(P.x + (size_t)m0 * K, K, wv, c1 - m0, xb[wv], lane);
-        } else {
-#pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                const int kb = wv * QK_K + kslot_base<FMT>(t, grp);
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) {
-                    const int m = m0 + nt * 16 + col;
-                    bx[t][nt] = load_x8<__half>(P.x + (size_t)(m < c1 ? m : c0) * K + kb, m < c1);
-                }
-            }
-        }
-    };
+    auto load_b = [&](int m0) { sb_stage_x(P.x + (size_t)m0 * K, K, wv, c1 - m0, xb[wv], lane); };
     load_b(c0);
     for (int m0 = c0; m0 < c1; m0 += 16 * NT) {
         floatx4_t acc[RT][NT];
@@ -311,12 +294,11 @@ __device__ __forceinline__ void mm_ws_body(const MmPlan& P, const MmTile& T, MfW
         for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) acc[rt][nt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-        if constexpr (NT == 1) {
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's copies; no other wave reads them
-            sb_read_x<FMT>(xb[wv], col, grp, bx);
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read: the next columns may land
-            if (m0 + 16 < c1) load_b(m0 + 16);
-        }
+        half8_t bx[8][NT];
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's copies; no other wave reads them
+        sb_read_x<FMT>(xb[wv], col, grp, bx);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read: the next columns may land
+        if (m0 + 16 < c1) load_b(m0 + 16);
         XMin<NT, XM> xm;
         sb_xmin<FMT, NT, XM>(bx, L[wv].xl, xm);
 #pragma unroll
@@ -327,22 +309,21 @@ __device__ __forceinline__ void mm_ws_body(const MmPlan& P, const MmTile& T, MfW
             for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) L[wv].red[rt][nt][i][lane] = acc[rt][nt][i];
-        if (NT > 1 && m0 + 16 * NT < c1) load_b(m0 + 16 * NT);
         __syncthreads();
         mm_epilogue<RT, NT, NW>(P, T, L, m0, min(16 * NT, c1 - m0));
         __syncthreads();
     }
 }
 
-template <int RT, int NT>
+template <int RT>
 __global__ __launch_bounds__(64 * 6) void fused_mm_ws_kernel(MmPlan P, int cols) {
-    __shared__ MfWave<RT, NT, false> L[6];
-    __shared__ alignas(16) _Float16 xb[NT == 1 ? 6 : 1][16 * QK_K];
+    __shared__ MfWave<RT, 1, false> L[6];
+    __shared__ alignas(16) _Float16 xb[6][16 * QK_K];
     const MmTile T = mm_tile<RT>(P, blockIdx.x);
     const int c0 = blockIdx.y * cols, c1 = min(P.M, c0 + cols);
     if (c0 >= c1) return;
-    if (T.S->fmt == 4) mm_ws_body<4, RT, NT>(P, T, L, xb, c0, c1);
-    else mm_ws_body<6, RT, NT>(P, T, L, xb, c0, c1);
+    if (T.S->fmt == 4) mm_ws_body<4, RT>(P, T, L, xb, c0, c1);
+    else mm_ws_body<6, RT>(P, T, L, xb, c0, c1);
 }
 
 // Eight SwiGLU outputs of column m from the sums of eight gate and up rows.
@@ -447,9 +428,9 @@ static int mm_env(const char* name, int dflt) {
 // Launch form of a batch of B columns, `tiles` 32-row tiles in all.  Above 32
 // columns at K = 6 super-blocks the tiled form where its blocks (of 32 columns
 // here) fill the chip, else the weight-stationary one, whose six waves each
-// take a super-block (q/k/v of 2048 rows, 40 / 256 / 512 columns: 7.9 / 13.3 /
-// 20.8 us against 18.9 / 19.1 / 22.4 tiled; gate/up of 17920 rows, 64 / 512
-// columns: 28.3 / 114 against 18.1 / 58.1); other K as in mt_beats_launches.
+// take a super-block (q/k/v of 2048 rows, 40 / 256 / 512 columns: 6.6 / 11.7 /
+// 17.6 us against 18.9 / 19.1 / 22.4 tiled; gate/up of 17920 rows, 64 / 512
+// columns: 28.3 / 114 against 17.2 / 53.3); other K as in mt_beats_launches.
 // VTE_MM_WS=0 selects the 32-column launches for every batch.
 enum MmForm { MM_COLS32, MM_WS, MM_TILED };
 static MmForm mm_form(int B, int tiles, int K) {
@@ -497,20 +478,12 @@ static hipError_t mm_run(MmPlan P, int B, MmForm form, size_t out_ld_elems[MM_MA
     __half* vc0 = P.v_cache;
     bool q6 = false;
     for (int s = 0; s < P.nseg; ++s) q6 = q6 || P.seg[s].fmt != 4;
-    if constexpr (RT == 4) if (form == MM_WS) {
-        // 64 rows per block, 16 columns at a time: one block per CU
-        const int g = ws_column_groups(total, B, device_cus());
+    if constexpr (RT != 3) if (form == MM_WS) {
+        // 64 rows per block: one block per CU; fewer: two
+        const int g = ws_column_groups(total, B, (RT == 4 ? 1 : 2) * device_cus());
         const int cols = ((B + 31) / 32 + g - 1) / g * 32, gy = (B + cols - 1) / cols;
         P.M = B;
-        hipLaunchKernelGGL((fused_mm_ws_kernel<RT, 1>), dim3(total, gy), dim3(64 * 6), 0, st, P, cols);
-        return hipGetLastError();
-    }
-    if constexpr (RT <= 2) if (form == MM_WS) {
-        // two 6-wave blocks fit per CU
-        const int g = ws_column_groups(total, B, 2 * device_cus());
-        const int cols = ((B + 31) / 32 + g - 1) / g * 32, gy = (B + cols - 1) / cols;
-        P.M = B;
-        hipLaunchKernelGGL((fused_mm_ws_kernel<RT, 2>), dim3(total, gy), dim3(64 * 6), 0, st, P, cols);
+        hipLaunchKernelGGL((fused_mm_ws_kernel<RT>), dim3(total, gy), dim3(64 * 6), 0, st, P, cols);
         return hipGetLastError();
     }
     for (int m0 = 0; m0 < B; m0 += 32) {
@@ -553,9 +526,11 @@ hipError_t qkv_mm(const void* xn, const void* wq, const void* q_bias, int fmt_q,
                   const int* kv_offset, int kv_batch_stride, const void* rope_cos, const void* rope_sin, int B, int K,
                   int n_q, int n_kv, hipStream_t st) {
     const MmForm form = mm_form(B, (n_q + 2 * n_kv) * 4, K);
-    // weight-stationary: 64 rows per block from 129 columns (2048-token prefill in chunks of 512:
-    // 38.5 -> 37.2 ms; chunks of 64-128 are faster with 16)
-    const int RT = form == MM_TILED ? 2 : mm_env("VTE_MM_RT_QKV", form == MM_WS && B > 128 ? 4 : 1);
+    // weight-stationary: 16, 32 or 64 rows per block up to 64, 128 and more
+    // columns (2048 rows; 64 / 128 / 256 columns: 6.7 / 11.6 / 19.7 us with 16 rows,
+    // 8.1 / 8.3 / 14.6 with 32, 11.5 / 11.6 / 11.7 with 64)
+    const int ws_rt = B > 128 ? 4 : B > 64 ? 2 : 1;
+    const int RT = form == MM_TILED ? 2 : mm_env("VTE_MM_RT_QKV", form == MM_WS ? ws_rt : 1);
     MmPlan P;
     memset(&P, 0, sizeof(P));
     P.K = K;
