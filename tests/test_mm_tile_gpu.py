@@ -78,3 +78,21 @@ def test_splitk_tiled(hip, K, fmt, k, n, M, splits):
     assert np.array_equal(got.view(np.uint32), one.view(np.uint32))
     ref = dq.gemv(fmt, raw, n, k, x.astype(np.float32))
     assert rel_l2(got.sum(0, dtype=np.float64), ref) <= TOL
+
+
+@pytest.mark.parametrize("k,n,M,splits", [(1792, 1, 16, 0), (2304, 17, 3, 0), (8960, 301, 16, 0), (4096, 4101, 9, 0),
+                                          (8960, 1537, 16, 5), (2048, 33, 5, 8)])
+def test_q6k_weights_through_lds(hip, K, k, n, M, splits):
+    """Q6_K batches of at most 16 columns: super-blocks at every offset in a 16-byte chunk, ragged rows and waves."""
+    rng = np.random.default_rng(k + n)
+    raw = syn.random_matrix("q6_k", rng, n, k, balanced=True)
+    x = rng.standard_normal((M, k)).astype(np.float16)
+    y = empty(hip, (max(splits, 1), M, n), np.float32)
+    if splits:
+        K.gemm_mfma_splitk("q6_k", up(hip, x), up(hip, raw), y, M, k, n, splits, stream=hip.stream)
+    else:
+        K.gemm_mfma("q6_k", up(hip, x), up(hip, raw), y, M, k, n, in_dtype="f16", out_dtype="f32", stream=hip.stream)
+    got, ref = down(y).sum(axis=0), dq.gemv("q6_k", raw, n, k, x.astype(np.float32))
+    assert np.isfinite(got).all()
+    for m in range(M):
+        assert rel_l2(got[m], ref[m]) <= TOL, m

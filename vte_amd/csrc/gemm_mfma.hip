@@ -22,12 +22,14 @@
 #include "mm_tile.h"
 
 // Body of one block: row tile blockIdx.x, split `split` of `nsplit` (split-K
-// partial sums at y + split * split_stride).
-template <typename TI, typename TO, int FMT, int RT, int NT, int NW>
+// partial sums at y + split * split_stride).  WST (Q6_K, NT = 1): raw weights
+// through LDS too (wst: 16 RT rows a wave), see launch_tile.
+template <typename TI, typename TO, int FMT, int RT, int NT, int NW, bool WST>
 __device__ __forceinline__ void gemm_mfma_body(const TI* __restrict__ x, const uint8_t* __restrict__ w,
                                                TO* __restrict__ y, int M, int K, int N, const TO* __restrict__ bias,
                                                const TO* __restrict__ residual, float rs, size_t split_stride,
-                                               int split, int nsplit, MfWave<RT, NT, NT == 1>* L) {
+                                               int split, int nsplit, MfWave<RT, NT, NT == 1>* L,
+                                               uint8_t* wst) {
     constexpr bool XM = NT > 1;  // minimum-term form (q4_xmin)
 
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -52,10 +54,22 @@ __device__ __forceinline__ void gemm_mfma_body(const TI* __restrict__ x, const u
         if constexpr (NT == 1) {  // staged activations: coalesced, and fp16 holds no registers in flight
             sb_stage_x(x, K, sb, M, L[wv].x, lane);
             typename SbRaw<FMT>::Raw raw[RT];
+            if constexpr (WST) {
+                uint8_t* wl = wst + wv * (16 * RT * Q6_STAGE_ROW);
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the last super-block's reads
+                q6_stage_w<RT>(w, row_bytes, sb, row0, N, wl, lane);
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-                sb_load(w + (size_t)min(row0 + rt * 16 + col, N - 1) * row_bytes + (size_t)sb * bpr, grp, raw[rt]);
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                for (int rt = 0; rt < RT; ++rt) {
+                    const uint8_t* p = w + (size_t)min(row0 + rt * 16 + col, N - 1) * row_bytes + (size_t)sb * bpr;
+                    mt_raw(wl + (16 * rt + col) * Q6_STAGE_ROW + (reinterpret_cast<uintptr_t>(p) & 15), grp, raw[rt]);
+                }
+            } else {
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt)
+                    sb_load(w + (size_t)min(row0 + rt * 16 + col, N - 1) * row_bytes + (size_t)sb * bpr, grp, raw[rt]);
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            }
             sb_staged<RT>(raw, L[wv].x, col, grp, acc);
             continue;
         } else {
@@ -111,14 +125,15 @@ __device__ __forceinline__ void gemm_mfma_body(const TI* __restrict__ x, const u
 }
 
 // NW waves per block split K (6 when K = 1536: one super-block each).
-template <typename TI, typename TO, int FMT, int RT, int NT, int NW = MF_WAVES>
-__global__ __launch_bounds__(64 * NW, RT == 2 && NT == 1 ? 4 : 1) void gemm_mfma_kernel(const TI* __restrict__ x, const uint8_t* __restrict__ w,
+template <typename TI, typename TO, int FMT, int RT, int NT, int NW = MF_WAVES, bool WST = false>
+__global__ __launch_bounds__(64 * NW, RT == 2 && NT == 1 && !WST ? 4 : 1) void gemm_mfma_kernel(const TI* __restrict__ x, const uint8_t* __restrict__ w,
                                                         TO* __restrict__ y, int M, int K, int N,
                                                         const TO* __restrict__ bias, const TO* __restrict__ residual,
                                                         float rs, size_t split_stride) {
     __shared__ MfWave<RT, NT, NT == 1> L[NW];
-    gemm_mfma_body<TI, TO, FMT, RT, NT, NW>(x, w, y, M, K, N, bias, residual, rs, split_stride, (int)blockIdx.y,
-                                            (int)gridDim.y, L);
+    __shared__ alignas(16) uint8_t wst[WST ? NW * 16 * RT * Q6_STAGE_ROW : 16];
+    gemm_mfma_body<TI, TO, FMT, RT, NT, NW, WST>(x, w, y, M, K, N, bias, residual, rs, split_stride, (int)blockIdx.y,
+                                            (int)gridDim.y, L, wst);
 }
 
 // Batched MFMA GEMM behind the reference GEMV's 10-argument ABI (fp16 I/O,
@@ -137,10 +152,10 @@ __device__ __forceinline__ void gemm_ref_abi(const void* input_ptr, const void* 
     const __half* x = static_cast<const __half*>(input_ptr) + (size_t)c0 * in_features;
     __half* y = static_cast<__half*>(output_ptr) + (size_t)c0 * out_features;
     const __half* res = residual_ptr ? static_cast<const __half*>(residual_ptr) + (size_t)c0 * out_features : nullptr;
-    gemm_mfma_body<__half, __half, FMT, 2, 1, MF_WAVES>(x, static_cast<const uint8_t*>(weight_ptr), y,
+    gemm_mfma_body<__half, __half, FMT, 2, 1, MF_WAVES, false>(x, static_cast<const uint8_t*>(weight_ptr), y,
                                                         min(16, cols - c0), in_features, out_features,
                                                         static_cast<const __half*>(bias_ptr), res, residual_scale, 0,
-                                                        0, 1, L);
+                                                        0, 1, L, nullptr);
 }
 extern "C" __global__ __launch_bounds__(64 * MF_WAVES) void gemm_q4k_mfma_kernel(
     const void* input_ptr, const void* weight_ptr, void* output_ptr, int batch, int seq_len, int in_features,
@@ -424,6 +439,19 @@ template <typename TI, typename TO, int FMT, int RT, int NT>
 static void launch_tile(const TI* x, const void* w, TO* y, int M, int K, int N, const void* bias,
                         const TO* residual, float rs, hipStream_t st, int splits = 1, size_t split_stride = 0) {
     const dim3 g((N + 16 * RT - 1) / (16 * RT), splits);
+    // Q6_K rows are 210 bytes a super-block, so a lane's 16-byte loads straddle
+    // lines and a wave's touch 16 rows: through LDS they are whole lines.  One
+    // block per CU then (16 columns; 10.6 -> 9.0 us for 8960 -> 1536 in 5 splits,
+    // 15.1 -> 9.1 us unsplit, 4096 -> 4096 10.7 -> 8.0 us), so only while every
+    // block has a CU: past that two resident blocks are faster
+    // (3072 -> 12000 14.2 us against 15.4).  A wave with one super-block hides
+    // the raw loads behind the activations' already (K = 1536, below).
+    if constexpr (FMT == 6 && NT == 1 && RT <= 2)
+        if (K > 6 * QK_K && (int)(g.x * g.y) <= device_cus()) {
+            hipLaunchKernelGGL((gemm_mfma_kernel<TI, TO, FMT, RT, NT, MF_WAVES, true>), g, dim3(64 * MF_WAVES), 0, st,
+                               x, (const uint8_t*)w, y, M, K, N, (const TO*)bias, residual, rs, split_stride);
+            return;
+        }
     if (K == 6 * QK_K && splits == 1)
         hipLaunchKernelGGL((gemm_mfma_kernel<TI, TO, FMT, RT, NT, 6>), g, dim3(64 * 6), 0, st, x, (const uint8_t*)w, y,
                            M, K, N, (const TO*)bias, residual, rs, split_stride);

@@ -388,6 +388,59 @@ struct alignas(16) MfWave {
     float xl[ST ? 4 : NT * 128];
 };
 
+#define MT_GLOBAL(p) ((const __attribute__((address_space(1))) void*)(p))
+#define MT_SHARED(p) ((__attribute__((address_space(3))) void*)(p))
+
+// 16 (or 8) bytes at a 2-byte aligned LDS address.
+template <int N>
+__device__ __forceinline__ void lds_words(const uint8_t* p, uint32_t (&v)[N]) {
+    const uint32_t a = (uint32_t)(uintptr_t)MT_SHARED(p);
+    const uint32_t* q = reinterpret_cast<const uint32_t*>(p - (a & 2));
+    uint32_t w[N + 1];
+#pragma unroll
+    for (int i = 0; i <= N; ++i) w[i] = q[i];
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = __builtin_amdgcn_alignbyte(w[i + 1], w[i], a & 2);
+}
+// A lane's raw bytes of its row's super-block from the staged copy.
+__device__ __forceinline__ void mt_raw(const uint8_t* blk, int grp, Q4Raw& r) { q4_raw_load(blk, grp, r); }
+__device__ __forceinline__ void mt_raw(const uint8_t* blk, int grp, Q6Raw& r) {
+    const int h = grp >> 1, j = grp & 1;
+    uint32_t a[4], b[4], c[4], s[2], d[1];
+    lds_words<4>(blk + 64 * h + 16 * j, a);
+    lds_words<4>(blk + 64 * h + 32 + 16 * j, b);
+    lds_words<4>(blk + 128 + 32 * h + 16 * j, c);
+    lds_words<2>(blk + 192 + 8 * h, s);
+    d[0] = *reinterpret_cast<const uint16_t*>(blk + 208);
+    r.la = make_uint4(a[0], a[1], a[2], a[3]);
+    r.lb = make_uint4(b[0], b[1], b[2], b[3]);
+    r.hq = make_uint4(c[0], c[1], c[2], c[3]);
+    r.sc = make_uint2(s[0], s[1]);
+    r.d = d[0];
+}
+
+
+// RT row tiles' raw Q6_K bytes of super-block sb (row r at w + r * row_bytes,
+// rows from n_rows on: the last) into a wave's LDS, 14 16-byte chunks a row from
+// the aligned-down start (a super-block's 210 bytes start 0..14 past it; every
+// chunk holds a byte of it), then each lane's share.  LDS-direct loads write a
+// lane's chunk at 16 * lane, so the copy is wlds[row * 224 + chunk * 16].
+#define Q6_STAGE_ROW 224
+template <int RT>
+__device__ __forceinline__ void q6_stage_w(const uint8_t* w, size_t row_bytes, int sb, int row0, int n_rows,
+                                           uint8_t* wlds, int lane) {
+    constexpr int CH = Q6_STAGE_ROW / 16, TOTAL = RT * 16 * CH;
+#pragma unroll
+    for (int j = 0; j < (TOTAL + 63) / 64; ++j) {
+        const int idx = j * 64 + lane, r = idx / CH, c = idx % CH;
+        const uintptr_t p = reinterpret_cast<uintptr_t>(w + (size_t)min(row0 + r, n_rows - 1) * row_bytes +
+                                                        (size_t)sb * Q6K_BYTES);
+        if (idx < TOTAL)
+            __builtin_amdgcn_global_load_lds(MT_GLOBAL((p & ~(uintptr_t)15) + 16 * c), MT_SHARED(wlds + j * 1024), 16,
+                                             0, 0);
+    }
+}
+
 // 16 columns' activations of super-block sb into a wave's LDS as fp16 rows of
 // 256, 16-byte chunks permuted by chunk ^ column so an operand read's 16
 // columns lie in distinct banks; columns past M stay as they are (results

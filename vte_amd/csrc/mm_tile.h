@@ -53,9 +53,6 @@ struct alignas(16) MtLds {
     };
 };
 
-#define MT_GLOBAL(p) ((const __attribute__((address_space(1))) void*)(p))
-#define MT_SHARED(p) ((__attribute__((address_space(3))) void*)(p))
-
 // Activations of super-block sb, columns c0 .. c0 + 16 NT - 1 (past M: column
 // M - 1, results unused), into LDS.  A wave's load fills two rows.  Where all
 // columns exist the row advance is scalar and a lane keeps two offsets.
@@ -142,34 +139,6 @@ __device__ __forceinline__ void mt_add(const Q6Ops& o, const floatx4_t& aw, cons
         const float t = o.d * aw[i];
         acc[i] = acc[i] + t;
     }
-}
-
-// 16 (or 8) bytes at a 2-byte aligned LDS address.
-template <int N>
-__device__ __forceinline__ void lds_words(const uint8_t* p, uint32_t (&v)[N]) {
-    const uint32_t a = (uint32_t)(uintptr_t)MT_SHARED(p);
-    const uint32_t* q = reinterpret_cast<const uint32_t*>(p - (a & 2));
-    uint32_t w[N + 1];
-#pragma unroll
-    for (int i = 0; i <= N; ++i) w[i] = q[i];
-#pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = __builtin_amdgcn_alignbyte(w[i + 1], w[i], a & 2);
-}
-// A lane's raw bytes of its row's super-block from the staged copy.
-__device__ __forceinline__ void mt_raw(const uint8_t* blk, int grp, Q4Raw& r) { q4_raw_load(blk, grp, r); }
-__device__ __forceinline__ void mt_raw(const uint8_t* blk, int grp, Q6Raw& r) {
-    const int h = grp >> 1, j = grp & 1;
-    uint32_t a[4], b[4], c[4], s[2], d[1];
-    lds_words<4>(blk + 64 * h + 16 * j, a);
-    lds_words<4>(blk + 64 * h + 32 + 16 * j, b);
-    lds_words<4>(blk + 128 + 32 * h + 16 * j, c);
-    lds_words<2>(blk + 192 + 8 * h, s);
-    d[0] = *reinterpret_cast<const uint16_t*>(blk + 208);
-    r.la = make_uint4(a[0], a[1], a[2], a[3]);
-    r.lb = make_uint4(b[0], b[1], b[2], b[3]);
-    r.hq = make_uint4(c[0], c[1], c[2], c[3]);
-    r.sc = make_uint2(s[0], s[1]);
-    r.d = d[0];
 }
 
 // Sums of a wave's two row tiles over super-blocks sb0 .. sb1 - 1 for the
