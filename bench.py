@@ -200,7 +200,7 @@ def mfma_b16_roofline(hip, ex, reps=20):
             traffic = json.load(f).get("hbm_bytes_per_launch")
     return {"bound": "hbm", "achieved": round(gbps, 1), "peak": HBM_PEAK_GBPS, "unit": "GB/s",
             "frac": round(gbps / HBM_PEAK_GBPS, 4), "traffic": traffic,
-            "kernel": "fused_mm_kernel<2, 1, 6> (gate/up + SwiGLU on MFMA, 28 launches of the batch-16 step)",
+            "kernel": "fused_mm_kernel<2, 1, 6, false> (gate/up + SwiGLU on MFMA, 28 launches of the batch-16 step)",
             "avg_launch_us": round(ms * 1e3, 3), "algo_bytes_per_launch": int(algo),
             "timing": "HIP events around graph replays of the step's 28 gate/up launches"}
 

@@ -80,8 +80,8 @@ int vte_gemm_mfma(int fmt, int in_dtype, int out_dtype, const void* x, const voi
                   int N, const void* bias, const void* residual, float residual_scale, void* stream);
 
 /* Split-K partial sums for batched projections (M >= 3; above 32 columns with
- * at most 8 super-blocks per split one weight-stationary launch, same
- * results), Q4_K / Q6_K, fp16 x:
+ * at most 8 super-blocks per split one tiled or weight-stationary launch, by
+ * size, same results), Q4_K / Q6_K, fp16 x:
  *   part[s][m][n] = sum over split s's super-blocks of dequant(W[n, k]) * x[m, k]
  * (fp32, no bias / scale / residual; 1 <= splits <= 8 and splits <= K / 256).
  * vte_add_rmsnorm adds the splits to the residual.
@@ -231,8 +231,8 @@ int vte_topk_exclude(const float* logits, int rows, int vocab, int k, float* out
  * or Q6_K.  norm_w NULL: x is already normalised (fp16) and is used as is.
  * With norm_w: batch 1..4 on the VALU mat-vec (norm fused in).  NULL norm_w:
  * batch 1..2 on the VALU mat-vec, batch 3..4096 on MFMA (launches of 32
- * sequences; above 32 one weight-stationary launch, same results); above
- * batch 4 norm_w must be NULL (RMSNorm runs before).
+ * sequences; above 32 one weight-stationary or tiled launch, by size, same
+ * results for hidden = 1536); above batch 4 norm_w must be NULL (RMSNorm runs before).
  * Replaces: the rmsnorm -> q/k/v gemv -> rope -> kv_cache_append nodes
  *           (vte/compiler/qwen_compute.py:100-282) and their fused forms
  *           FusedQKVDispatcher (vte/core/fused_qkv_dispatch.py:12-198),
@@ -246,7 +246,8 @@ int vte_attn_in(const void* x, const void* norm_w, float eps, const void* wq, co
 /* One launch: RMSNorm(x) -> gate and up projections -> fp16(silu(g) * u),
  * out [B][ffn], Q4_K gate/up.  norm_w NULL: x is already normalised.
  * With norm_w: batch 1..4 on the VALU mat-vec.  NULL norm_w: batch 1..2 on
- * the VALU mat-vec, 3..4096 on MFMA; above batch 4 norm_w must be NULL.
+ * the VALU mat-vec, 3..4096 on MFMA (above 32 one tiled or
+ * weight-stationary launch, by size); above batch 4 norm_w must be NULL.
  * Replaces: FusedFFNDispatcher (vte/core/fused_qkv_dispatch.py:200-270) with
  *           fused_gate_up_silu_kernel (fused_rmsnorm_gate_up_silu.hip.template:66-111). */
 int vte_ffn_in(const void* x, const void* norm_w, float eps, const void* w_gate, const void* w_up, int fmt,
