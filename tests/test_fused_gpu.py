@@ -191,6 +191,30 @@ def test_ffn_in_batched_mfma(hip, K, B, ffn):
         assert np.array_equal(down(out).view(np.uint16), got.view(np.uint16))
 
 
+@pytest.mark.parametrize("B", [3, 20, 40, 130])
+def test_ffn_in_mfma_swiglu_precision(hip, K, B):
+    """SwiGLU of the MFMA launches (one and two column tiles, tiled) on gates of a few tens: each result within one fp16
+    rounding and the fp32 bound of exp (one unit), 1 + e, the division and the product (half a unit each, 2.5 units of
+    2^-23, taken as 3) of the value in 64 bits.  The gate and up values are the plain GEMM's, the same bits."""
+    k, ffn = 1536, 8960
+    rng = np.random.default_rng(B)
+    wg, wu = (syn.random_matrix("q4_k", rng, ffn, k, balanced=True) for _ in range(2))
+    x = (8 * rng.standard_normal((B, k))).astype(np.float16)
+    dx, dg, du = up(hip, x), up(hip, wg), up(hip, wu)
+    g, u = empty(hip, (B, ffn), np.float16), empty(hip, (B, ffn), np.float16)
+    for w, y in ((dg, g), (du, u)):
+        K.gemm_mfma("q4_k", dx, w, y, B, k, ffn, in_dtype="f16", out_dtype="f16", stream=hip.stream)
+    out = empty(hip, (B, ffn), np.float16)
+    K.ffn_in(dx, None, EPS, dg, du, "q4_k", out, B, k, ffn, stream=hip.stream)
+    g, u = down(g).astype(np.float64), down(u).astype(np.float64)
+    assert (g < -8).sum() > 1000
+    ref = g / (1 + np.exp(-g)) * u
+    normal = (np.abs(ref) >= 2.0 ** -14) & (np.abs(ref) < 65504)
+    got, ref = down(out).astype(np.float64)[normal], ref[normal]
+    half = 2.0 ** (np.floor(np.log2(np.abs(ref))) - 11)
+    assert (np.abs(got - ref) <= half + 3 * 2.0 ** -23 * np.abs(ref)).all()
+
+
 def test_batch_above_4_rejects_fused_norm(hip, K):
     """The MFMA path takes normalised activations: passing norm weights is an error."""
     import ctypes

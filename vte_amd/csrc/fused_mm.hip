@@ -187,10 +187,11 @@ __device__ __forceinline__ float mm_sum(const MfWave<RT, NT, ST>* L, int rr, int
 
 __device__ __forceinline__ float mm_bias(const __half* b, int row) { return b ? __half2float(b[row]) : 0.f; }
 
-// g / (1 + e^-g) with the hardware's exponential and reciprocal: a few fp32
-// units off, under an fp16 rounding; the library forms are about 30
-// instructions per output (gate/up of 512 columns 57.4 -> 55.0 us without them).
-__device__ __forceinline__ float mm_silu(float g) { return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)); }
+// g / (1 + e^-g) with the library's exponential and a division, as every other
+// SwiGLU of the decode path.  The hardware's exponential and reciprocal are
+// faster (gate/up of 512 columns of 8960: 53.1 against 54.9 us), but several
+// fp32 units off for gates of -8 and below, which flips fp16 results.
+__device__ __forceinline__ float mm_silu(float g) { return g / (1.0f + expf(-g)); }
 
 // Epilogue of one output (row, batch column m of the launch: position
 // kv_offset[m], row m of the outputs) from its sum.
