@@ -327,3 +327,42 @@ def test_prompt_chunk_attention(hip, K, B, offsets, n_q, n_kv, split, dtype):
             p = np.exp(s - s.max())
             ref = p @ vc[:n, h // (n_q // n_kv)].astype(np.float64) / p.sum()
             assert rel_l2(got[b, h], ref) <= TOL, (b, h)
+
+
+def _prompt_run(hip, K, q, kc, vc, off, n_q, n_kv, split=128, one_cache=True):
+    """vte_attn_split_kv of len(off) columns over one cache kc/vc [rows][n_kv][D]."""
+    B, ms = len(off), -(-kc.shape[0] // split)
+    pm, pl = empty(hip, (B, n_q, ms), np.float32), empty(hip, (B, n_q, ms), np.float32)
+    po, out = empty(hip, (B, n_q, ms, D), np.float32), empty(hip, (B, n_q, D), q.dtype)
+    K.attn_split_kv(up(hip, q), up(hip, kc), up(hip, vc), pm, pl, po, out, B, n_q, n_kv, D, SCALE, up(hip, off), 0,
+                    split, ms, dtype="f32" if q.dtype == np.float32 else "f16", stream=hip.stream)
+    return down(out)
+
+
+@pytest.mark.parametrize("B,offsets,n_q,n_kv,dtype", [(130, "run", 12, 2, "f16"), (65, "run", 2, 2, "f32"),
+                                                      (200, "any", 7, 1, "f32"), (70, "first", 8, 1, "f16")])
+def test_prompt_chunk_values_of_later_positions(hip, K, B, offsets, n_q, n_kv, dtype):
+    """Inf and NaN in V rows that some columns of a block see and others do not: they reach the results of the columns
+    at and past their position, in their own dimension, and no other result."""
+    rng = np.random.default_rng(B)
+    off = {"run": np.arange(250, 250 + B), "any": rng.integers(0, 600, B),
+           "first": np.minimum(np.arange(B), 40)}[offsets].astype(np.int32)
+    q = rng.standard_normal((B, n_q, D)).astype(np.float32 if dtype == "f32" else np.float16)
+    kc, vc = (rng.standard_normal((700, n_kv, D)).astype(np.float16) for _ in range(2))
+    order = np.sort(off)
+    bad = [(int(order[5]), 0, 3, np.inf), (int(order[B // 2]), n_kv - 1, 17, np.nan), (int(order[B // 2]), 0, 64, -np.inf),
+           (int(order[-1]), 0, 127, np.nan), (int(order[B // 3]), n_kv - 1, 90, np.inf)]
+    for pos, kv, d, v in bad:
+        vc[pos, kv, d] = v
+    vc[off.max() + 1:] = np.inf
+    got = _prompt_run(hip, K, q, kc, vc, off, n_q, n_kv).astype(np.float64)
+    for b in range(B):
+        n = int(off[b]) + 1
+        for h in range(n_q):
+            kv = h // (n_q // n_kv)
+            s = kc[:n, kv].astype(np.float64) @ q[b, h].astype(np.float16).astype(np.float64) * SCALE
+            w = np.exp(s - s.max())
+            ref = w @ vc[:n, kv].astype(np.float64) / w.sum()
+            same = np.isfinite(ref)
+            assert np.array_equal(got[b, h][~same], ref[~same], equal_nan=True), (b, h)
+            assert rel_l2(got[b, h][same], ref[same]) <= TOL, (b, h)

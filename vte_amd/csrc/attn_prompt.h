@@ -11,7 +11,11 @@
 // loads, the next 64 tokens' under this step's products), scores are K.Q^T
 // (lane = row, so the softmax state is per lane), the probabilities are the
 // A operand of P.V as they stand, and V's operand comes from the transposing
-// LDS read.  The tokens up to the block's longest column are cut into nsp
+// LDS read.  A wave stops at its own longest row.  In the steps where rows of
+// the block end, tokens past a row have probability 0, and 0 * Inf and 0 * NaN
+// are NaN: when such a step leaves a non-finite sum, its products are formed
+// again by ap_pv_masked, which multiplies a row only with the tokens it sees
+// (the check is 32 fmas; reading the V tile for it took 1 us).  The tokens up to the block's longest column are cut into nsp
 // equal shares, one per grid.z, so every block of a launch does about the same
 // work wherever the chunk lies in the prompt; the shares' partial results meet
 // in attn_prompt_combine.
@@ -21,6 +25,8 @@
 // the LDS reads but leave one wave per SIMD: 24.5 against 23.0 us (512 columns
 // of 12 heads after 1536 rows), 15.8 against 13.3 (128 columns).
 #pragma once
+#include <type_traits>
+
 #include "attn_tile.h"
 
 #define AP_ROWS 64  // rows of a block
@@ -66,6 +72,38 @@ __device__ __forceinline__ void ap_stage(ApTile& T, const __half* kb, const __ha
     }
 }
 
+// Whether any lane's sums hold an Inf or a NaN (the same answer in every lane).
+__device__ __forceinline__ bool ap_nonfinite(const floatx4_t (&o)[ATT_D / 16]) {
+    float z[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int dt = 0; dt < ATT_D / 16; ++dt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) z[i] = fmaf(o[dt][i], 0.f, z[i]);
+    return __any(!((z[0] + z[1]) + (z[2] + z[3]) == 0.f));
+}
+
+// o += P.V on the vector units, row 4 grp + i over its first cnt[i] tokens only
+// (rare: see above).  e[tt][i]: probability of row col, token 16 tt + 4 grp + i.
+__device__ __forceinline__ void ap_pv_masked(const ApTile& T, const floatx4_t (&e)[4], const int (&cnt)[4],
+                                             floatx4_t (&o)[ATT_D / 16], int lane) {
+    const int col = lane & 15, grp = lane >> 4;
+#pragma unroll 1
+    for (int t = 0; t < AP_TOK; ++t) {
+        float ev = e[0][0];
+#pragma unroll
+        for (int j = 1; j < 16; ++j) ev = (4 * (t >> 4) + (t & 3)) == j ? e[j >> 2][j & 3] : ev;
+        float pr[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) pr[i] = __shfl(ev, 4 * grp + i + 16 * ((t >> 2) & 3), 64);
+#pragma unroll
+        for (int dt = 0; dt < ATT_D / 16; ++dt) {
+            const float v = (float)T.v[t * ATT_D + 8 * ((2 * dt + (col >> 3)) ^ (2 * (t & 7))) + (col & 7)];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[dt][i] = t < cnt[i] ? fmaf(pr[i], v, o[dt][i]) : o[dt][i];
+        }
+    }
+}
+
 // grid (row blocks, n_kv, nsp), block 256.  max_ctx: rows of the cache that
 // may be read.  nsp == 1: out holds the results; else part_m / part_l / part_o
 // [n_cols][n_q][max_splits] (x 128) hold share z's at index z < nsp.
@@ -75,7 +113,7 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(
     float* __restrict__ part_m, float* __restrict__ part_l, float* __restrict__ part_o, TO* __restrict__ out, int n_q,
     int n_kv, float scale, const int* __restrict__ kv_offset, int n_cols, int max_ctx, int max_splits) {
     __shared__ ApTile tile[2];
-    __shared__ int red[ATT_WAVES];
+    __shared__ int red[2][ATT_WAVES];
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, grp = lane >> 4;
     const int G = n_q / n_kv, kvh = blockIdx.y, sp = blockIdx.z, nsp = gridDim.z;
@@ -84,7 +122,7 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(
     const __half* kb = k_cache + (size_t)kvh * ATT_D;
     const __half* vb = v_cache + (size_t)kvh * ATT_D;
 
-    // this lane's row: query operands and length; the wave's shortest and the block's longest length
+    // this lane's row: query operands and length; the wave's longest length, the block's shortest and longest
     half8_t qb[ATT_D / 32];
     int len;
     {
@@ -99,12 +137,17 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(
         longest = max(longest, __shfl_xor(longest, i, 64));
         shortest = min(shortest, __shfl_xor(shortest, i, 64));
     }
-    shortest = __builtin_amdgcn_readfirstlane(shortest);
-    if (lane == 0) red[wv] = longest;
+    longest = __builtin_amdgcn_readfirstlane(longest);
+    if (lane == 0) {
+        red[0][wv] = longest;
+        red[1][wv] = shortest;
+    }
     __syncthreads();
-    const int total = __builtin_amdgcn_readfirstlane(max(max(red[0], red[1]), max(red[2], red[3])));
+    const int total = __builtin_amdgcn_readfirstlane(max(max(red[0][0], red[0][1]), max(red[0][2], red[0][3])));
     const int share = ((total + nsp - 1) / nsp + AP_TOK - 1) / AP_TOK * AP_TOK;
     const int t_begin = sp * share, t_end = min(total, t_begin + share);
+    const int all_end = __builtin_amdgcn_readfirstlane(
+        min(min(min(red[1][0], red[1][1]), min(red[1][2], red[1][3])), t_end));  // every row reaches this far
 
     const float c2 = scale * 1.44269504088896340736f;  // exp(scale s) = 2^(c2 s)
     float m_run = -1e30f, l_run = 0.f;  // raw score maximum of the row; this lane's share of its sum
@@ -125,10 +168,9 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
     }
-    int cur = 0;
-    for (int t0 = t_begin; t0 < t_end; t0 += AP_TOK, cur ^= 1) {
-        const ApTile& T = tile[cur];
-        if (t0 + AP_TOK < t_end) ap_stage(tile[cur ^ 1], kb, vb, row_stride, t0 + AP_TOK, t_end - 1, wv, lane);
+    // One step over tile T.  ENDS: some row of the block ends in it (or the share does).
+    auto step = [&](const ApTile& T, int t0, auto ends) {
+        constexpr bool ENDS = decltype(ends)::value;
         // ---- scores: lane holds S[row col][token 16 tt + 4 grp + i] ----
         floatx4_t s[4];
 #pragma unroll
@@ -140,7 +182,7 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(
                     *reinterpret_cast<const half8_t*>(T.k + 16 * tt * ATT_D + ko[d]), qb[d], s[tt], 0, 0, 0);
         }
         // ---- online softmax ----
-        if (t0 + AP_TOK > min(shortest, t_end)) {  // some row ends in this step (or the share does)
+        if constexpr (ENDS) {
             const int end = min(len, t_end) - t0 - 4 * grp;
 #pragma unroll
             for (int tt = 0; tt < 4; ++tt)
@@ -171,10 +213,15 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(
         for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const float e = __builtin_amdgcn_exp2f(fmaf(s[tt][i], c2, mc));
-                l_run += e;
-                p[tt >> 1][4 * (tt & 1) + i] = (_Float16)e;
+                s[tt][i] = __builtin_amdgcn_exp2f(fmaf(s[tt][i], c2, mc));
+                l_run += s[tt][i];
+                p[tt >> 1][4 * (tt & 1) + i] = (_Float16)s[tt][i];
             }
+        floatx4_t before[ATT_D / 16];
+        if constexpr (ENDS) {
+#pragma unroll
+            for (int dt = 0; dt < ATT_D / 16; ++dt) before[dt] = o[dt];
+        }
         // ---- P.V: V[token slots][dim 16 dt + col] by transposing reads of 4 tokens x 16 dims ----
 #pragma unroll
         for (int u = 0; u < 2; ++u)
@@ -190,8 +237,36 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(
                         (__attribute__((address_space(3))) ap_s4*)(T.v + (2 * u + e) * 16 * ATT_D + vo[dt]));
                 o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(p[u], vf.v, o[dt], 0, 0, 0);
             }
+        if constexpr (ENDS) {
+            if (ap_nonfinite(o)) {
+                int cnt[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) cnt[i] = min(__shfl(len, 4 * grp + i, 64), t_end) - t0;
+#pragma unroll
+                for (int dt = 0; dt < ATT_D / 16; ++dt) o[dt] = before[dt];
+                ap_pv_masked(T, s, cnt, o, lane);
+            }
+        }
+    };
+    int t0 = t_begin, cur = 0;
+    auto stage_next = [&] {
+        if (t0 + AP_TOK < t_end) ap_stage(tile[cur ^ 1], kb, vb, row_stride, t0 + AP_TOK, t_end - 1, wv, lane);
+    };
+    auto next = [&] {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the next tokens' copies
         __syncthreads();
+        t0 += AP_TOK;
+        cur ^= 1;
+    };
+    while (t0 + AP_TOK <= all_end) {
+        stage_next();
+        step(tile[cur], t0, std::false_type{});
+        next();
+    }
+    while (t0 < t_end) {
+        stage_next();
+        if (t0 < longest) step(tile[cur], t0, std::true_type{});  // past its rows a wave only takes part in the copies
+        next();
     }
 
     // ---- results: rows 4 grp + i of the wave's tile ----
