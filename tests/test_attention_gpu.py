@@ -366,3 +366,29 @@ def test_prompt_chunk_values_of_later_positions(hip, K, B, offsets, n_q, n_kv, d
             same = np.isfinite(ref)
             assert np.array_equal(got[b, h][~same], ref[~same], equal_nan=True), (b, h)
             assert rel_l2(got[b, h][same], ref[same]) <= TOL, (b, h)
+
+
+@pytest.mark.parametrize("spread", [0.5, 3.0, 8.0])
+def test_prompt_chunk_precision(hip, K, spread):
+    """The 64-row blocks are no further from the 64-bit result than the decode path's form (one column per block), over
+    flat and peaked score distributions (standard deviations 0.5 to 8), fp32 results."""
+    import os
+    rng = np.random.default_rng(3)
+    B, n_q, n_kv, rows = 128, 4, 1, 1500
+    off = np.arange(rows - B, rows, dtype=np.int32)
+    q = (2 * spread * rng.standard_normal((B, n_q, D))).astype(np.float16).astype(np.float32)
+    kc, vc = (0.5 * rng.standard_normal((rows, n_kv, D)).astype(np.float16) for _ in range(2))
+    got = _prompt_run(hip, K, q, kc, vc, off, n_q, n_kv)
+    os.environ["VTE_ATT_QC"] = "0"
+    try:
+        one = _prompt_run(hip, K, q, kc, vc, off, n_q, n_kv)
+    finally:
+        del os.environ["VTE_ATT_QC"]
+    ref = np.empty(q.shape)
+    for b in range(B):
+        n = int(off[b]) + 1
+        s = q[b].astype(np.float64) @ kc[:n, 0].astype(np.float64).T * SCALE
+        w = np.exp(s - s.max(axis=1, keepdims=True))
+        ref[b] = w @ vc[:n, 0].astype(np.float64) / w.sum(axis=1, keepdims=True)
+    assert not np.array_equal(got, one)
+    assert rel_l2(got, ref) <= rel_l2(one, ref)

@@ -20,10 +20,11 @@
 // work wherever the chunk lies in the prompt; the shares' partial results meet
 // in attn_prompt_combine.
 //
-// Bound by instruction issue: per 16 rows and 64 tokens 32 MFMAs (512 matrix
-// cycles) stand beside about 180 other instructions.  32 rows per wave halve
+// Bound by instruction issue: per 16 rows and 64 tokens 48 MFMAs (768 matrix
+// cycles) stand beside about 300 other instructions.  32 rows per wave halve
 // the LDS reads but leave one wave per SIMD: 24.5 against 23.0 us (512 columns
-// of 12 heads after 1536 rows), 15.8 against 13.3 (128 columns).
+// of 12 heads after 1536 rows, probabilities in one part), 15.8 against 13.3
+// (128 columns).
 #pragma once
 #include <type_traits>
 
@@ -32,6 +33,23 @@
 #define AP_ROWS 64  // rows of a block
 #define AP_TOK 64   // tokens of a step
 #define AP_MAX_SPLITS 8
+
+// Probabilities are held as 2^14 exp(score - running maximum) and enter P.V as
+// two fp16 parts, hi (rounded down) and lo (the rest): about 21 bits down to
+// 2^-38 of the maximum.  One fp16 part relative to a whole share's maximum was
+// up to twice as far from the 64-bit result as the other forms, whose reference
+// is a 32-token tile's (fp32 results, 1500 rows, scores of standard deviation
+// 0.5 / 8: 2.0e-4 / 1.8e-5 against 1.8e-4 / 0.9e-5; two parts 3.4e-7 / 7.0e-7).
+// The second part costs 16 MFMAs a step (512 columns after 1536 rows: 21.5 ->
+// 23.0 us).  lo's last bit is set, so both parts of a seen token are positive and
+// Inf in V stays Inf (0 * Inf is NaN).
+#define AP_P_LOG2 14.0f
+typedef __fp16 ap_h2 __attribute__((ext_vector_type(2)));
+union ApP {
+    half8_t v;
+    ap_h2 h[4];
+    uint32_t u[4];
+};
 
 typedef short ap_s4 __attribute__((ext_vector_type(4)));
 typedef unsigned ap_u2 __attribute__((ext_vector_type(2)));
@@ -149,6 +167,8 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(
     const int all_end = __builtin_amdgcn_readfirstlane(
         min(min(min(red[1][0], red[1][1]), min(red[1][2], red[1][3])), t_end));  // every row reaches this far
 
+    float neg1 = -1.f;
+    asm volatile("" : "+v"(neg1));  // keeps a - hi one mixed-precision fma (a conversion and a subtraction else)
     const float c2 = scale * 1.44269504088896340736f;  // exp(scale s) = 2^(c2 s)
     float m_run = -1e30f, l_run = 0.f;  // raw score maximum of the row; this lane's share of its sum
     floatx4_t o[ATT_D / 16];            // rows 4 grp + i, dim 16 dt + col
@@ -207,16 +227,23 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(
 #pragma unroll
                 for (int i = 0; i < 4; ++i) o[dt][i] *= cr[i];
         }
-        const float mc = -mx * c2;
-        half8_t p[2];
+        const float mc = fmaf(-mx, c2, AP_P_LOG2);
 #pragma unroll
         for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 s[tt][i] = __builtin_amdgcn_exp2f(fmaf(s[tt][i], c2, mc));
                 l_run += s[tt][i];
-                p[tt >> 1][4 * (tt & 1) + i] = (_Float16)s[tt][i];
             }
+        ApP hi[2], lo[2];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float a = s[j >> 1][2 * (j & 1)], b = s[j >> 1][2 * (j & 1) + 1];
+            const ap_h2 h = __builtin_amdgcn_cvt_pkrtz(a, b);
+            hi[j >> 2].h[j & 3] = h;
+            lo[j >> 2].h[j & 3] = __builtin_amdgcn_cvt_pkrtz(fmaf((float)h[0], neg1, a), fmaf((float)h[1], neg1, b));
+            if constexpr (!ENDS) lo[j >> 2].u[j & 3] |= 0x00010001u;
+        }
         floatx4_t before[ATT_D / 16];
         if constexpr (ENDS) {
 #pragma unroll
@@ -224,19 +251,23 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(
         }
         // ---- P.V: V[token slots][dim 16 dt + col] by transposing reads of 4 tokens x 16 dims ----
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int u = 0; u < 2; ++u) {
+            union {
+                ap_s4 h[2];
+                half8_t v;
+            } vf[ATT_D / 16];
 #pragma unroll
             for (int dt = 0; dt < ATT_D / 16; ++dt) {
-                union {
-                    ap_s4 h[2];
-                    half8_t v;
-                } vf;
 #pragma unroll
                 for (int e = 0; e < 2; ++e)
-                    vf.h[e] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    vf[dt].h[e] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                         (__attribute__((address_space(3))) ap_s4*)(T.v + (2 * u + e) * 16 * ATT_D + vo[dt]));
-                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(p[u], vf.v, o[dt], 0, 0, 0);
+                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[u].v, vf[dt].v, o[dt], 0, 0, 0);
             }
+#pragma unroll
+            for (int dt = 0; dt < ATT_D / 16; ++dt)
+                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo[u].v, vf[dt].v, o[dt], 0, 0, 0);
+        }
         if constexpr (ENDS) {
             if (ap_nonfinite(o)) {
                 int cnt[4];
