@@ -392,3 +392,19 @@ def test_prompt_chunk_precision(hip, K, spread):
         ref[b] = w @ vc[:n, 0].astype(np.float64) / w.sum(axis=1, keepdims=True)
     assert not np.array_equal(got, one)
     assert rel_l2(got, ref) <= rel_l2(one, ref)
+
+
+@pytest.mark.parametrize("B,start,n_q,n_kv,split", [(100, 290, 4, 1, 128), (130, 0, 12, 2, 128), (70, 330, 7, 1, 32)])
+def test_prompt_chunk_bits_do_not_depend_on_the_capacity(hip, K, B, start, n_q, n_kv, split):
+    """The token shares of a chunk follow from its positions: the same bits in caches of any capacity of 1024 rows and
+    more.  Smaller ones allow fewer shares: fp32 rounding apart."""
+    rng = np.random.default_rng(B)
+    off = np.arange(start, start + B, dtype=np.int32)
+    q = rng.standard_normal((B, n_q, D)).astype(np.float32)
+    kc, vc = (rng.standard_normal((4000, n_kv, D)).astype(np.float16) for _ in range(2))
+    ref = _prompt_run(hip, K, q, kc, vc, off, n_q, n_kv, split)
+    for rows in (start + B, 640, 1024, 1700):
+        got = _prompt_run(hip, K, q, kc[:rows], vc[:rows], off, n_q, n_kv, split)
+        if rows >= 1024:
+            assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), rows
+        assert rel_l2(got, ref) <= 2e-6, rows  # two parts of a probability: 2^-21, and fp32 sums

@@ -494,9 +494,14 @@ static hipError_t attn_prompt(const void* q, const void* k_cache, const void* v_
                               float* part_o, void* out, int B, int n_q, int n_kv, float scale, const int* kv_offset,
                               int max_ctx, int max_splits, hipStream_t st) {
     // token shares: as many as two blocks per CU hold (512 columns of 12 heads,
-    // 2048 rows: 256 / 512 / 768 blocks 30.5 / 23.0 / 25.9 us), of 128 rows at least
+    // 2048 rows: 256 / 512 / 768 blocks 30.5 / 23.0 / 25.9 us), and no more than
+    // the capacity has 128-row pieces and the partial results have places.  The
+    // positions are on the device, so a short prompt in a large cache leaves some
+    // shares empty; its shares are then 64 rows (at least 128 would make the count
+    // independent of capacities below 1024 rows too, but takes 8.0 -> 9.1 us for 65
+    // columns at start 0, 9.5 -> 11.1 for 200).
     const int rbs = (B * (n_q / n_kv) + AP_ROWS - 1) / AP_ROWS;
-    const int nsp = std::max(1, std::min({AP_MAX_SPLITS, max_splits, max_ctx / 128, 512 / (rbs * n_kv)}));
+    const int nsp = std::max(1, std::min({AP_MAX_SPLITS, max_splits, max_ctx / 128, 2 * device_cus() / (rbs * n_kv)}));
     hipLaunchKernelGGL((attn_prompt_kernel<TQ, TO>), dim3(rbs, n_kv, nsp), dim3(256), 0, st, (const TQ*)q,
                        (const __half*)k_cache, (const __half*)v_cache, part_m, part_l, part_o, (TO*)out, n_q, n_kv,
                        scale, kv_offset, B, max_ctx, max_splits);

@@ -15,10 +15,10 @@
 // the block end, tokens past a row have probability 0, and 0 * Inf and 0 * NaN
 // are NaN: when such a step leaves a non-finite sum, its products are formed
 // again by ap_pv_masked, which multiplies a row only with the tokens it sees
-// (the check is 32 fmas; reading the V tile for it took 1 us).  The tokens up to the block's longest column are cut into nsp
-// equal shares, one per grid.z, so every block of a launch does about the same
-// work wherever the chunk lies in the prompt; the shares' partial results meet
-// in attn_prompt_combine.
+// (the check is 32 fmas; reading the V tile for it took 1 us).  The tokens up to
+// the block's longest column are cut into nsp equal shares, one per grid.z, so
+// every block of a launch does about the same work wherever the chunk lies in
+// the prompt; the shares' partial results meet in attn_prompt_combine.
 //
 // Bound by instruction issue: per 16 rows and 64 tokens 48 MFMAs (768 matrix
 // cycles) stand beside about 300 other instructions.  32 rows per wave halve

@@ -565,14 +565,3 @@ static inline int ws_column_groups(int tiles, int M, int slots) {
     }
     return best;
 }
-
-// Compute units of the current device (cached after the first query).
-static inline int device_cus() {
-    static int n = 0;
-    if (n == 0) {
-        int dev = 0;
-        (void)hipGetDevice(&dev);
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    }
-    return n;
-}

@@ -104,3 +104,14 @@ __device__ __forceinline__ void gemv_store(TO* out, const TO* bias, const TO* re
     if (residual) acc += ld_act<TO>(residual + o);
     st_act<TO>(out + o, acc);
 }
+
+// Compute units of the current device (cached after the first query).
+static inline int device_cus() {
+    static int n = 0;
+    if (n == 0) {
+        int dev = 0;
+        (void)hipGetDevice(&dev);
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    }
+    return n;
+}
