@@ -298,7 +298,6 @@ __device__ __forceinline__ void mm_ws_body(const MmPlan& P, const MmTile& T, MfW
         half8_t bx[8][NT];
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's copies; no other wave reads them
         sb_read_x<FMT>(xb[wv], col, grp, bx);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read: the next columns may land
         if (m0 + 16 < c1) load_b(m0 + 16);
         XMin<NT, XM> xm;
         sb_xmin<FMT, NT, XM>(bx, L[wv].xl, xm);

@@ -224,7 +224,6 @@ __global__ __launch_bounds__(64 * MF_WAVES) void gemm_ws_splitk_kernel(const __h
             half8_t bx[8][NT];
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's copies; no other wave reads them
             sb_read_x<FMT>(xb[wv], col, grp, bx);
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read: the next columns may land
             if (m0 + 16 < c1) load_b(m0 + 16);
             XMin<NT, XM> xm;
             sb_xmin<FMT, NT, XM>(bx, xl[wv], xm);

@@ -445,9 +445,11 @@ __device__ __forceinline__ void q6_stage_w(const uint8_t* w, size_t row_bytes, i
 // 256, 16-byte chunks permuted by chunk ^ column so an operand read's 16
 // columns lie in distinct banks; columns past M stay as they are (results
 // unused).  Consecutive lanes take consecutive bytes, and fp16 goes straight
-// to LDS, holding no registers (wait for vmcnt before reading it).
+// to LDS, holding no registers (wait for vmcnt before reading it).  The copy
+// waits for the wave's reads of what it overwrites (their products have been
+// issued by then, so the wait is free).
 __device__ __forceinline__ void sb_stage_x(const __half* x, int K, int sb, int M, _Float16* lds, int lane) {
-    asm volatile("" : "+v"(lane));  // addresses made here, not kept across the loop over super-blocks
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(lane)::"memory");  // (and addresses made here, not kept across the loop)
     const int hi = lane >> 5, slot = lane & 31;
     const char* base = reinterpret_cast<const char*>(x + sb * QK_K);
 #pragma unroll
