@@ -1,5 +1,7 @@
 """The tiled MFMA GEMM of batches above 32 columns at its edges: last row tiles, last column tiles, every column-tile
 width, formats whose rows straddle 16-byte chunks, K other than the weight-stationary kernel's, unaligned outputs."""
+import os
+
 import numpy as np
 import pytest
 
@@ -58,7 +60,6 @@ def test_ffn_in_tiled(hip, K, k, ffn, B):
                                               ("q6_k", 8960, 1500, 200, 7), ("q4_k", 256, 9000, 512, 1)])
 def test_splitk_tiled(hip, K, fmt, k, n, M, splits):
     """Split-K partial sums of the tiled form: the bits of the 32-column launches."""
-    import os
     rng = np.random.default_rng(k + M)
     raw = syn.random_matrix(fmt, rng, n, k, balanced=True)
     x = rng.standard_normal((M, k)).astype(np.float16)
@@ -96,3 +97,71 @@ def test_q6k_weights_through_lds(hip, K, k, n, M, splits):
     assert np.isfinite(got).all()
     for m in range(M):
         assert rel_l2(got[m], ref[m]) <= TOL, m
+
+
+@pytest.mark.parametrize("k,n_q,n_kv,B,fmt_v,bias", [
+    (512, 4, 1, 100, "q6_k", True), (512, 7, 1, 515, "q4_k", True), (256, 3, 3, 65, "q6_k", False),
+    (2048, 5, 1, 129, "q6_k", True), (2048, 12, 2, 333, "q4_k", False),
+    (1536, 12, 2, 515, "q6_k", True), (1536, 28, 4, 257, "q4_k", True),
+    (1536, 12, 2, 65, "q6_k", True), (1536, 4, 2, 128, "q4_k", True)])
+def test_attn_in_above_32_columns(hip, K, k, n_q, n_kv, B, fmt_v, bias):
+    """q/k/v + bias + RoPE + K/V rows in the tiled form (hidden sizes other than 1536, long batches of it, Q4_K and Q6_K
+    rows in one launch) and in the weight-stationary form of 32 rows per block: against the oracle, the bits of the
+    32-column launches (a wave there owns at most one super-block), and no other cache row written."""
+    hd, max_seq = 128, 700
+    rng = np.random.default_rng(k + B)
+    wq, wk = (syn.random_matrix("q4_k", rng, n * hd, k, balanced=True) for n in (n_q, n_kv))
+    wv = syn.random_matrix(fmt_v, rng, n_kv * hd, k, balanced=True)
+    b = [(0.5 * rng.standard_normal(n * hd)).astype(np.float16) for n in (n_q, n_kv, n_kv)]
+    x = rng.standard_normal((B, k)).astype(np.float16)
+    pos = rng.permutation(max_seq)[:B].astype(np.int32)
+    cos_c, sin_c = ost.rope_cache(max_seq, hd, 1e6)
+    dx, dq_, dk, dv, dpos, dc, ds = (up(hip, a) for a in (x, wq, wk, wv, pos, cos_c, sin_c))
+    db = [up(hip, a) if bias else None for a in b]
+
+    def run():
+        q, kc, vc = (empty(hip, s, np.float16) for s in ((B, n_q * hd), (max_seq, n_kv, hd), (max_seq, n_kv, hd)))
+        K.attn_in(dx, None, 1e-6, dq_, db[0], "q4_k", dk, db[1], "q4_k", dv, db[2], fmt_v, q, kc, vc, dpos, 0, dc, ds, B,
+                  k, n_q, n_kv, stream=hip.stream)  # stride 0: the columns are positions of one sequence
+        return down(q), down(kc), down(vc)
+
+    got = run()
+    os.environ["VTE_MM_WS"] = "0"
+    try:
+        one = run()
+    finally:
+        del os.environ["VTE_MM_WS"]
+    for a, c in zip(got, one):
+        assert np.array_equal(a.view(np.uint16), c.view(np.uint16))
+    x32 = x.astype(np.float32)
+    ref = [dq.gemv(f, w, n * hd, k, x32) + (bb.astype(np.float32) if bias else 0)
+           for f, w, n, bb in (("q4_k", wq, n_q, b[0]), ("q4_k", wk, n_kv, b[1]), (fmt_v, wv, n_kv, b[2]))]
+    ref = [r.astype(np.float16).reshape(B, -1, hd) for r in ref]
+    for m, p in enumerate(pos):
+        assert rel_l2(got[0][m], ost.rope_neox(ref[0][m], p, cos_c, sin_c).reshape(-1)) <= TOL, m
+        assert rel_l2(got[1][p], ost.rope_neox(ref[1][m], p, cos_c, sin_c)) <= TOL, m
+        assert rel_l2(got[2][p], ref[2][m]) <= TOL, m
+    others = np.delete(np.arange(max_seq), pos)
+    assert not got[1][others].any() and not got[2][others].any()
+
+
+@pytest.mark.parametrize("fmt", ["q4_k", "q6_k"])
+@pytest.mark.parametrize("n,k,M", [(8961, 2048, 40), (1000, 1536, 515), (4100, 768, 96)])
+def test_gemm_tiled_bits(hip, K, fmt, n, k, M):
+    """vte_gemm_mfma tiled: the bits of the 32-column launches where a wave of those owns at most one super-block."""
+    rng = np.random.default_rng(n)
+    raw = syn.random_matrix(fmt, rng, n, k, balanced=True)
+    dx, dw = up(hip, rng.standard_normal((M, k)).astype(np.float16)), up(hip, raw)
+
+    def run():
+        y = empty(hip, (M, n), np.float32)
+        K.gemm_mfma(fmt, dx, dw, y, M, k, n, in_dtype="f16", out_dtype="f32", stream=hip.stream)
+        return down(y)
+
+    got = run()
+    os.environ["VTE_MM_WS"] = "0"
+    try:
+        one = run()
+    finally:
+        del os.environ["VTE_MM_WS"]
+    assert np.array_equal(got.view(np.uint32), one.view(np.uint32))
