@@ -165,3 +165,24 @@ def test_gemm_tiled_bits(hip, K, fmt, n, k, M):
     finally:
         del os.environ["VTE_MM_WS"]
     assert np.array_equal(got.view(np.uint32), one.view(np.uint32))
+
+
+@pytest.mark.parametrize("fmt", ["q4_k", "q6_k"])
+@pytest.mark.parametrize("k,n,M,splits", [(256, 17, 3, 1), (1024, 4100, 16, 1), (768, 1537, 5, 2), (2048, 1000, 8, 8),
+                                          (1792, 555, 16, 2), (1280, 40, 9, 1)])
+def test_splitk_few_super_blocks(hip, K, fmt, k, n, M, splits):
+    """At most 16 columns with up to four super-blocks per split (four-wave blocks), uneven shares, and five (eight waves):
+    every split's sums against the oracle over its super-blocks."""
+    rng = np.random.default_rng(k + n)
+    raw = syn.random_matrix(fmt, rng, n, k, balanced=True)
+    x = rng.standard_normal((M, k)).astype(np.float16)
+    y = empty(hip, (splits, M, n), np.float32)
+    K.gemm_mfma_splitk(fmt, up(hip, x), up(hip, raw), y, M, k, n, splits, stream=hip.stream)
+    got, sb = down(y), k // 256
+    blocks = raw.reshape(n, sb, -1)
+    for s in range(splits):
+        a, b = sb * s // splits, sb * (s + 1) // splits
+        ref = dq.gemv(fmt, np.ascontiguousarray(blocks[:, a:b]).reshape(-1), n, 256 * (b - a),
+                      x[:, 256 * a:256 * b].astype(np.float32))
+        for m in range(M):
+            assert rel_l2(got[s, m], ref[m]) <= 1e-5, (s, m)  # fp32 sums of exact products

@@ -451,6 +451,16 @@ static void launch_tile(const TI* x, const void* w, TO* y, int M, int K, int N, 
                                x, (const uint8_t*)w, y, M, K, N, (const TO*)bias, residual, rs, split_stride);
             return;
         }
+    // At most four super-blocks to a split: four waves hold them, and half the
+    // staging LDS lets four blocks share a CU instead of two (three columns, blocks
+    // above two per CU: 2048 -> 1536 in 8 splits 5.1 -> 3.8 us).  The four idle
+    // waves' sums would be zero, so the bits are the same.
+    if constexpr (NT == 1 && RT <= 2)
+        if ((K / QK_K + splits - 1) / splits <= 4) {
+            hipLaunchKernelGGL((gemm_mfma_kernel<TI, TO, FMT, RT, NT, 4>), g, dim3(64 * 4), 0, st, x,
+                               (const uint8_t*)w, y, M, K, N, (const TO*)bias, residual, rs, split_stride);
+            return;
+        }
     if (K == 6 * QK_K && splits == 1)
         hipLaunchKernelGGL((gemm_mfma_kernel<TI, TO, FMT, RT, NT, 6>), g, dim3(64 * 6), 0, st, x, (const uint8_t*)w, y,
                            M, K, N, (const TO*)bias, residual, rs, split_stride);
