@@ -224,6 +224,29 @@ def test_reference_abi_mfma_symbol(hip, name, fmt, k, cols):
     assert rel_l2(down(y), ref) <= TOL
 
 
+@pytest.mark.parametrize("name,fmt", [("gemm_q4k_mfma_kernel", "q4_k"), ("gemm_q6k_mfma_kernel", "q6_k")])
+@pytest.mark.parametrize("offset", [1, 4])
+def test_reference_abi_mfma_symbol_input_alignment(hip, name, fmt, offset):
+    """The input may start at any fp16 element: same bits as an aligned copy (partial row and column tiles)."""
+    from vte_amd.kernels import HSACO_PATH
+    _, fn = hip.load_kernel(str(HSACO_PATH), name)
+    n, k, cols = 50, 2304, 19
+    rng = np.random.default_rng(offset)
+    raw = syn.random_matrix(fmt, rng, n, k)
+    x = rng.standard_normal(cols * k).astype(np.float16)
+    dw, got = up(hip, raw), []
+    for off in (0, offset):
+        dx, y = up(hip, np.concatenate([np.zeros(off, np.float16), x])), empty(hip, (cols, n), np.float16)
+        args = [ctypes.c_void_p(dx.ptr + 2 * off), ctypes.c_void_p(dw.ptr), ctypes.c_void_p(y.ptr), ctypes.c_int(cols),
+                ctypes.c_int(1), ctypes.c_int(k), ctypes.c_int(n), ctypes.c_void_p(None), ctypes.c_void_p(None),
+                ctypes.c_float(1.0)]
+        hip.launch_kernel(fn, ((n + 31) // 32, (cols + 15) // 16, 1), (512, 1, 1), args, expected_args=10)
+        got.append(down(y))
+    assert np.array_equal(got[0].view(np.uint16), got[1].view(np.uint16))
+    ref = dq.gemv(fmt, raw, n, k, x.reshape(cols, k).astype(np.float32))
+    assert rel_l2(got[0], ref) <= TOL
+
+
 @pytest.mark.parametrize("fmt,n,k", [("q4_k", 37, 8960), ("q6_k", 29, 1536), ("q8_0", 11, 2048)])
 def test_measurement_read_kernel(hip, fmt, n, k):
     """The benchmark's read baseline (vte_read_rows_kernel, one 64-thread

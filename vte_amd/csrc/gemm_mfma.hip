@@ -23,8 +23,9 @@
 
 // Body of one block: row tile blockIdx.x, split `split` of `nsplit` (split-K
 // partial sums at y + split * split_stride).  WST (Q6_K, NT = 1): raw weights
-// through LDS too (wst: 16 RT rows a wave), see launch_tile.
-template <typename TI, typename TO, int FMT, int RT, int NT, int NW, bool WST>
+// through LDS too (wst: 16 RT rows a wave), see launch_tile.  XANY: fp16 x of
+// any alignment (NT = 1).
+template <typename TI, typename TO, int FMT, int RT, int NT, int NW, bool WST, bool XANY = false>
 __device__ __forceinline__ void gemm_mfma_body(const TI* __restrict__ x, const uint8_t* __restrict__ w,
                                                TO* __restrict__ y, int M, int K, int N, const TO* __restrict__ bias,
                                                const TO* __restrict__ residual, float rs, size_t split_stride,
@@ -52,7 +53,8 @@ __device__ __forceinline__ void gemm_mfma_body(const TI* __restrict__ x, const u
 
     for (int sb = sb0; sb < sb1; ++sb) {
         if constexpr (NT == 1) {  // staged activations: coalesced, and fp16 holds no registers in flight
-            sb_stage_x(x, K, sb, M, L[wv].x, lane);
+            if constexpr (XANY) sb_stage_x_any(x, K, sb, M, L[wv].x, lane);
+            else sb_stage_x(x, K, sb, M, L[wv].x, lane);
             typename SbRaw<FMT>::Raw raw[RT];
             if constexpr (WST) {
                 uint8_t* wl = wst + wv * (16 * RT * Q6_STAGE_ROW);
@@ -152,10 +154,13 @@ __device__ __forceinline__ void gemm_ref_abi(const void* input_ptr, const void* 
     const __half* x = static_cast<const __half*>(input_ptr) + (size_t)c0 * in_features;
     __half* y = static_cast<__half*>(output_ptr) + (size_t)c0 * out_features;
     const __half* res = residual_ptr ? static_cast<const __half*>(residual_ptr) + (size_t)c0 * out_features : nullptr;
-    gemm_mfma_body<__half, __half, FMT, 2, 1, MF_WAVES, false>(x, static_cast<const uint8_t*>(weight_ptr), y,
-                                                        min(16, cols - c0), in_features, out_features,
-                                                        static_cast<const __half*>(bias_ptr), res, residual_scale, 0,
-                                                        0, 1, L, nullptr);
+#define GEMM_REF_BODY(XANY_)                                                                                        \
+    gemm_mfma_body<__half, __half, FMT, 2, 1, MF_WAVES, false, XANY_>(                                                  \
+        x, static_cast<const uint8_t*>(weight_ptr), y, min(16, cols - c0), in_features, out_features,                   \
+        static_cast<const __half*>(bias_ptr), res, residual_scale, 0, 0, 1, L, nullptr)
+    if ((reinterpret_cast<uintptr_t>(input_ptr) & 15) == 0) GEMM_REF_BODY(false);
+    else GEMM_REF_BODY(true);
+#undef GEMM_REF_BODY
 }
 extern "C" __global__ __launch_bounds__(64 * MF_WAVES) void gemm_q4k_mfma_kernel(
     const void* input_ptr, const void* weight_ptr, void* output_ptr, int batch, int seq_len, int in_features,

@@ -460,6 +460,18 @@ __device__ __forceinline__ void sb_stage_x(const __half* x, int K, int sb, int M
                                          (__attribute__((address_space(3))) void*)(lds + 2 * j * QK_K), 16, 0, 0);
     }
 }
+// The same through registers, for rows of any alignment (the reference-ABI
+// symbols take any pointer; an LDS-direct load wants an aligned one).
+__device__ __forceinline__ void sb_stage_x_any(const __half* x, int K, int sb, int M, _Float16* lds, int lane) {
+    const int hi = lane >> 5, slot = lane & 31;
+    uint4 v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+        v[j] = q6_ld16(reinterpret_cast<const uint8_t*>(x + (size_t)min(2 * j + hi, M - 1) * K + sb * QK_K +
+                                                        8 * (slot ^ (2 * j + hi))));
+#pragma unroll
+    for (int j = 0; j < 8; ++j) *reinterpret_cast<uint4*>(lds + 2 * j * QK_K + 8 * lane) = v[j];
+}
 __device__ __forceinline__ void sb_stage_x(const float* x, int K, int sb, int M, _Float16* lds, int lane) {
     typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
     float4 v[16];
