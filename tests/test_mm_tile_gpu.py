@@ -102,13 +102,13 @@ def test_q6k_weights_through_lds(hip, K, k, n, M, splits):
 @pytest.mark.parametrize("k,n_q,n_kv,B,fmt_v,bias", [
     (512, 4, 1, 100, "q6_k", True), (512, 7, 1, 515, "q4_k", True), (256, 3, 3, 65, "q6_k", False),
     (2048, 5, 1, 129, "q6_k", True), (2048, 12, 2, 333, "q4_k", False),
-    (1536, 12, 2, 515, "q6_k", True), (1536, 28, 4, 257, "q4_k", True),
+    (1536, 12, 2, 801, "q6_k", True), (1536, 28, 4, 385, "q4_k", True),
     (1536, 12, 2, 65, "q6_k", True), (1536, 4, 2, 128, "q4_k", True)])
 def test_attn_in_above_32_columns(hip, K, k, n_q, n_kv, B, fmt_v, bias):
     """q/k/v + bias + RoPE + K/V rows in the tiled form (hidden sizes other than 1536, long batches of it, Q4_K and Q6_K
     rows in one launch) and in the weight-stationary form of 32 rows per block: against the oracle, the bits of the
     32-column launches (a wave there owns at most one super-block), and no other cache row written."""
-    hd, max_seq = 128, 700
+    hd, max_seq = 128, 900
     rng = np.random.default_rng(k + B)
     wq, wk = (syn.random_matrix("q4_k", rng, n * hd, k, balanced=True) for n in (n_q, n_kv))
     wv = syn.random_matrix(fmt_v, rng, n_kv * hd, k, balanced=True)

@@ -426,18 +426,25 @@ static int mm_env(const char* name, int dflt) {
 }
 
 // Launch form of a batch of B columns, `tiles` 32-row tiles in all.  Above 32
-// columns at K = 6 super-blocks the tiled form where its blocks (of 32 columns
-// here) fill the chip, else the weight-stationary one, whose six waves each
-// take a super-block (q/k/v of 2048 rows, 40 / 256 / 512 columns: 6.6 / 11.7 /
-// 17.6 us against 18.9 / 19.1 / 22.4 tiled; gate/up of 17920 rows, 64 / 512
-// columns: 28.3 / 114 against 17.2 / 53.3); other K as in mt_beats_launches.
+// columns at K = 6 super-blocks the weight-stationary form, whose six waves each
+// take a super-block, while its column groups are few: q/k/v up to 1.5 blocks of
+// the tiled form (128 rows x 32 columns) per CU, gate/up up to half a block (its
+// blocks hold twice the rows).  q/k/v of 2048 rows, 512 / 768 / 1024 columns 17.4 /
+// 22.2 / 29.8 us against 20.0 / 25.1 / 28.5 tiled, of 4608 rows, 256 / 384 columns
+// 22.1 / 26.8 against 23.9 / 25.4; gate/up of 2 x 2000 rows, 128 / 160 / 384 columns
+// 9.8 / 13.6 / 18.2 against 12.9 / 12.8 / 17.6, of 2 x 8960, 64 columns 24.3 against
+// 17.4.  Both forms give the same bits there.  Other K as in mt_beats_launches.
 // VTE_MM_WS=0 selects the 32-column launches for every batch.
 enum MmForm { MM_COLS32, MM_WS, MM_TILED };
-static MmForm mm_form(int B, int tiles, int K) {
+static MmForm mm_form(int B, int tiles, int K, bool swiglu) {
     if (B <= 32 || mm_env("VTE_MM_WS", 1) == 0) return MM_COLS32;
-    const int row_blocks = (tiles + MT_WAVES - 1) / MT_WAVES;
-    if (K == 6 * QK_K) return row_blocks * ((B + 31) / 32) < 258 ? MM_WS : MM_TILED;
-    return mt_beats_launches(row_blocks, B, K / QK_K, false) ? MM_TILED : MM_COLS32;
+    const int row_blocks = (tiles + MT_WAVES - 1) / MT_WAVES, cus = device_cus();
+    if (K == 6 * QK_K) return row_blocks * ((B + 31) / 32) <= (swiglu ? cus / 2 : cus + cus / 2) ? MM_WS : MM_TILED;
+    // (the launches' blocks: 24 pairs of gate/up rows, 16 rows of q/k/v; RoPE and
+    // the cache writes cost the tiled form more than the small blocks)
+    const MtCost cost = swiglu ? MtCost{3.9f, 1.55f, 5.1f, 0.3f, 0.008f} : MtCost{7.1f, 1.98f, 4.0f, 0.2f, 0.0105f};
+    return mt_beats_launches(row_blocks, swiglu ? (tiles * 2 + 2) / 3 : 2 * tiles, B, K / QK_K, cus, cost) ? MM_TILED
+                                                                                                          : MM_COLS32;
 }
 static hipError_t mm_run_tiled(MmPlan P, int B, hipStream_t st) {
     int total = 0;
@@ -525,7 +532,7 @@ hipError_t qkv_mm(const void* xn, const void* wq, const void* q_bias, int fmt_q,
                   int fmt_k, const void* wv, const void* v_bias, int fmt_v, void* q_out, void* k_cache, void* v_cache,
                   const int* kv_offset, int kv_batch_stride, const void* rope_cos, const void* rope_sin, int B, int K,
                   int n_q, int n_kv, hipStream_t st) {
-    const MmForm form = mm_form(B, (n_q + 2 * n_kv) * 4, K);
+    const MmForm form = mm_form(B, (n_q + 2 * n_kv) * 4, K, false);
     // weight-stationary: 16, 32 or 64 rows per block up to 64, 128 and more
     // columns (2048 rows; 64 / 128 / 256 columns: 6.7 / 11.6 / 19.7 us with 16 rows,
     // 8.1 / 8.3 / 14.6 with 32, 11.5 / 11.6 / 11.7 with 64)
@@ -559,7 +566,7 @@ hipError_t gate_up_mm(const void* xn, const void* w_gate, const void* w_up, int 
     // 16 gate/up pairs per block (half the blocks of 8, activations read half
     // as often); 24 for 17-32 columns (measured: batch 32 2.26 -> 2.18 ms per
     // step, batch 8-16 slightly slower); 32 in the weight-stationary form
-    const MmForm form = mm_form(B, (ffn + 15) / 16, K);
+    const MmForm form = mm_form(B, (ffn + 15) / 16, K, true);
     const int RT = form == MM_TILED ? 2 : mm_env("VTE_MM_RT_FFN", form == MM_WS ? 4 : B > 16 ? 3 : 2);
     MmPlan P;
     memset(&P, 0, sizeof(P));

@@ -5,7 +5,7 @@
 // Same contract as the GEMV (vte/compiler/templates/rdna/gemv_q4k.hip.template:56-168);
 // the reference re-reads W once per batch row (grid.y = batch), this kernel
 // reads it once per 32-column batch tile (above 32 columns once per column
-// group of up to 128, mm_tile.h).
+// group of up to 96, mm_tile.h).
 //
 // Design:
 //  * v_mfma_f32_16x16x32_f16 with exact integer weight operands and the
@@ -445,11 +445,12 @@ static void launch_tile(const TI* x, const void* w, TO* y, int M, int K, int N, 
     const dim3 g((N + 16 * RT - 1) / (16 * RT), splits);
     // Q6_K rows are 210 bytes a super-block, so a lane's 16-byte loads straddle
     // lines and a wave's touch 16 rows: through LDS they are whole lines.  One
-    // block per CU then (16 columns; 10.6 -> 9.0 us for 8960 -> 1536 in 5 splits,
-    // 15.1 -> 9.1 us unsplit, 4096 -> 4096 10.7 -> 8.0 us), so only while every
+    // block per CU then (16 columns; 8.3 -> 5.8 us for 8960 -> 1536 in 5 splits,
+    // 15.4 -> 9.2 us unsplit, 4096 -> 4096 10.6 -> 7.9 us), so only while every
     // block has a CU: past that two resident blocks are faster
-    // (3072 -> 12000 14.2 us against 15.4).  A wave with one super-block hides
-    // the raw loads behind the activations' already (K = 1536, below).
+    // (3584 -> 4096 in 2 splits, 6000 and more rows; up to twice the time with
+    // many blocks).  At K = 1536 the weights take one round trip beside the
+    // activations' either way: 4.5 -> 4.3 us, not worth another kernel there.
     if constexpr (FMT == 6 && NT == 1 && RT <= 2)
         if (K > 6 * QK_K && (int)(g.x * g.y) <= device_cus()) {
             hipLaunchKernelGGL((gemm_mfma_kernel<TI, TO, FMT, RT, NT, MF_WAVES, true>), g, dim3(64 * MF_WAVES), 0, st,
@@ -549,11 +550,13 @@ static hipError_t launch_tiled(const TI* x, const void* w, TO* y, int M, int K, 
 template <typename TI, typename TO, int FMT>
 static hipError_t launch_mfma(const void* x, const void* w, void* y, int M, int K, int N, const void* bias,
                               const void* residual, float rs, hipStream_t st) {
-    if (M > 32 && mt_beats_launches((N + MT_ROWS - 1) / MT_ROWS, M, K / QK_K, sizeof(TI) == 4) && !getenv_off("VTE_MM_WS"))
+    const bool tall = N >= 4096;
+    if (M > 32 && !getenv_off("VTE_MM_WS") &&
+        mt_beats_launches((N + MT_ROWS - 1) / MT_ROWS, tall ? (N + 31) / 32 : (N + 15) / 16, M, K / QK_K, device_cus(),
+                          mt_gemm_cost(FMT == 6, sizeof(TI) == 4, tall)))
         return launch_tiled<TI, TO, FMT>((const TI*)x, w, (TO*)y, M, K, N, (const TO*)bias, (const TO*)residual, rs, 1,
                                          st);
     if (K == GS_K && N >= 16384 && gs_lds_ok(M)) return launch_stream<TI, TO, FMT>(x, w, y, M, N, bias, residual, rs, st);
-    const bool tall = N >= 4096;
     for (int m0 = 0; m0 < M; m0 += 32) {
         const int mc = (M - m0 < 32) ? (M - m0) : 32;
         const TI* xs = (const TI*)x + (size_t)m0 * K;
@@ -583,12 +586,14 @@ static hipError_t launch_splitk(const void* x, const void* w, float* part, int M
     const int n_sb = K / QK_K;
     if (M > 32 && (n_sb + splits - 1) / splits <= MF_WAVES && !getenv_off("VTE_MM_WS")) {
         // The tiled form from 43 blocks (of 32 columns) per super-block of a
-        // split, which it takes one after another (2.7 us each) where this form
-        // gives each a wave: 8960 -> 1536 in 5 splits, 128 / 256 / 512 columns,
-        // Q6_K 24.7 / 35.7 / 58.0 us weight-stationary against 21.2 / 27.3 / 34.6
-        // tiled, Q4_K 19.6 / 31.3 / 55.2 against 19.9 / 27.8 / 34.9 (64 columns:
-        // 13.8 against 19.1); 1536 -> 1536 in 2 splits, 128 / 256 / 512 columns,
-        // 11.1 / 16.0 / 24.9 against 11.4 / 12.3 / 15.4 (with the add + norm launch).
+        // split, which it takes one after another where this form gives each a
+        // wave and pays per round of column groups.  8960 -> 1536 in 5 splits, 128 /
+        // 160 / 256 / 512 columns: Q6_K 17.6 / 20.7 / 24.1 / 36.4 us weight-stationary
+        // against 17.8 / 21.7 / 22.8 / 28.7 tiled, Q4_K 13.6 / 17.5 / 21.7 / 37.5
+        // against 15.8 / 20.3 / 21.7 / 29.1; 1536 -> 1536 in 2 splits, Q4_K, 128 / 200 /
+        // 256 columns: 7.1 / 10.2 / 10.3 against 8.3 / 8.4 / 8.9.  (The rounds are not
+        // in the rule: 5632 -> 2048 in 3 splits of Q6_K, 200 columns takes 30.1 where
+        // the tiled form would take 24.8.)
         const int tb = (N + MT_ROWS - 1) / MT_ROWS * splits * ((M + 31) / 32);
         if (tb >= 43 * ((n_sb + splits - 1) / splits))
             return launch_tiled<__half, float, FMT>((const __half*)x, w, part, M, K, N, nullptr, nullptr, 1.f, splits,

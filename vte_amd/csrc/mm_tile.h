@@ -315,10 +315,10 @@ static inline int mt_grid(int row_blocks, int groups) { return (row_blocks * gro
 
 // Column tiles per block.  Four decode a super-block for the fewest
 // instructions per column that still leave 8 waves per CU (gate/up of 17920
-// rows, 512 columns: 69.4 / 58.1 / 60.5 us with 2 / 4 / 6); two where four give
-// less than a block per CU (8960 -> 1536 in 5 splits, 128 columns: 21.2 against
-// 24.9 us); six where that saves a second round of two blocks per CU (gate/up,
-// 256 columns: 33.6 against 38.5 us).
+// rows, 512 columns: 67.5 / 57.0 / 58.3 us with 2 / 4 / 6); two where four give
+// less than a block per CU (8960 -> 1536 in 5 splits, Q4_K, 256 columns: 21.3
+// against 23.5 us); six where that saves a second round of two blocks per CU
+// (gate/up, 256 columns: 30.8 against 36.6 us).
 static inline int mt_pick_nt(int row_blocks, int splits, int M, int cus) {
     const auto blocks = [&](int nt) { return (long long)row_blocks * splits * ((M + 16 * nt - 1) / (16 * nt)); };
     if (blocks(4) < cus) return 2;
@@ -326,14 +326,25 @@ static inline int mt_pick_nt(int row_blocks, int splits, int M, int cus) {
 }
 
 // Whether one tiled launch beats a launch per 32 columns whose waves split K.
-// Always where its blocks (of 32 columns here) fill the chip; with fewer it
-// still takes the super-blocks one after another, about 1.9 us each, against
-// launches that grow with the columns (5 us and 0.4, fp32 activations 0.95, per
-// super-block and 32 columns): 8960 -> 1536, fp16, 40 / 64 columns 66 / 66 us
-// tiled against 35 / 47, fp32 75 / 75 against 59 / 79; q/k/v of 2048 rows, K =
-// 3584, 40 / 200 columns 35.5 / 40.9 against 20.9 / 168; K = 1536, 8960 rows,
-// fp32, 40 / 512 columns 14.9 / 46 against 32.6 / 332.
-static inline bool mt_beats_launches(int row_blocks, int M, int n_sb, bool f32) {
-    if ((long long)row_blocks * ((M + 31) / 32) >= 258) return true;
-    return 0.5 * ((M + 15) / 16) * (5.0 + (f32 ? 0.95 : 0.4) * n_sb) > 3.0 + 1.9 * n_sb;
+// Always where its blocks (of 32 columns here) outnumber the CUs.  With fewer it
+// still takes the super-blocks one after another, against launches that each
+// cost a start and grow with the super-blocks and their columns (and with the
+// rounds of their blocks): both linear, us, fitted to 3060 shapes of 33 to 200
+// columns, where the form picked is at most 1.12 times the other (mean 1.001).
+struct MtCost {
+    float tile, tile_sb;                   // tiled: a + b n_sb
+    float launch, launch_sb, launch_col;   // launches (c + d n_sb) + e n_sb M
+};
+// vte_gemm_mfma: Q6_K weights and fp32 activations take longer in either form;
+// tall: 32-row blocks in the launches.
+static inline MtCost mt_gemm_cost(bool q6, bool f32, bool tall) {
+    return MtCost{3.5f, 1.5f + (q6 ? 0.25f : 0.f) + (f32 ? 0.25f : 0.f),
+                  3.1f + (f32 ? 0.6f : 0.f) - (q6 ? 0.5f : 0.f) + (tall ? 0.55f : 0.f),
+                  q6 ? (tall ? 0.47f : 0.29f) : (tall ? 0.25f : 0.19f), f32 ? 0.022f : 0.011f};
+}
+static inline bool mt_beats_launches(int row_blocks, int launch_blocks, int M, int n_sb, int cus, const MtCost& c) {
+    const int launches = (M + 31) / 32;
+    if ((long long)row_blocks * launches > cus) return true;
+    const int rounds = (launch_blocks + cus - 1) / cus;
+    return rounds * (launches * (c.launch + c.launch_sb * n_sb) + c.launch_col * n_sb * M) > c.tile + c.tile_sb * n_sb;
 }
