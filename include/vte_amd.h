@@ -235,7 +235,7 @@ int vte_topk_exclude(const float* logits, int rows, int vocab, int k, float* out
  * With norm_w: batch 1..4 on the VALU mat-vec (norm fused in).  NULL norm_w:
  * batch 1..2 on the VALU mat-vec, batch 3..4096 on MFMA (launches of 32
  * sequences; above 32 one weight-stationary or tiled launch, by size, same
- * results for hidden = 1536); above batch 4 norm_w must be NULL (RMSNorm runs before).
+ * results for hidden up to 2048, fp32 rounding apart beyond); above batch 4 norm_w must be NULL (RMSNorm runs before).
  * Replaces: the rmsnorm -> q/k/v gemv -> rope -> kv_cache_append nodes
  *           (vte/compiler/qwen_compute.py:100-282) and their fused forms
  *           FusedQKVDispatcher (vte/core/fused_qkv_dispatch.py:12-198),
@@ -250,7 +250,8 @@ int vte_attn_in(const void* x, const void* norm_w, float eps, const void* wq, co
  * out [B][ffn], Q4_K gate/up.  norm_w NULL: x is already normalised.
  * With norm_w: batch 1..4 on the VALU mat-vec.  NULL norm_w: batch 1..2 on
  * the VALU mat-vec, 3..4096 on MFMA (above 32 one tiled or
- * weight-stationary launch, by size); above batch 4 norm_w must be NULL.
+ * weight-stationary launch, by size, results as for vte_attn_in); above batch 4
+ * norm_w must be NULL.
  * Replaces: FusedFFNDispatcher (vte/core/fused_qkv_dispatch.py:200-270) with
  *           fused_gate_up_silu_kernel (fused_rmsnorm_gate_up_silu.hip.template:66-111). */
 int vte_ffn_in(const void* x, const void* norm_w, float eps, const void* w_gate, const void* w_up, int fmt,

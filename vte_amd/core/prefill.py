@@ -6,10 +6,14 @@ docs/LIMITATIONS.md:11).  Here a chunk of C prompt tokens of sequence s is
 one batched step whose C columns are tokens of that same sequence: every
 column carries its own position, the q/k/v launch writes each column's K/V
 row into sequence s's cache at that position (sequence stride 0), and each
-column's split-KV attention reads the cache up to its own position, which
-is causal attention over the prompt.  Projections run on the MFMA kernels
-(C >= 8 columns per launch), so the weights are read once per 32 columns
-instead of once per token.  Only the last column goes through the LM head.
+column's attention reads the cache up to its own position, which is causal
+attention over the prompt.  Projections run on the MFMA kernels: above 32
+columns one tiled or weight-stationary launch each, so a weight is decoded
+once per 32 to 96 columns (or once per block of columns) instead of once per
+token.  Above 64 columns the attention runs in 64-row blocks whose results
+differ from the narrower chunks' by the fp16 rounding of the latter's
+probabilities, so K/V bits depend on which side of 64 a chunk's width lies.
+Only the last column goes through the LM head.
 
 A short last chunk runs at the smallest power of two (at least 4) that
 holds it, padded by repeating its last token at its position: the repeated

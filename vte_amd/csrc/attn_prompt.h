@@ -345,7 +345,7 @@ __global__ __launch_bounds__(256) void attn_prompt_combine(const float* __restri
         const int s = min(j, nsp - 1);
         m[j] = part_m[st + s];
         l[j] = part_l[st + s];
-        o[j] = *reinterpret_cast<const float4*>(part_o + (st + s) * ATT_D + d);
+        __builtin_memcpy(&o[j], part_o + (st + s) * ATT_D + d, sizeof(float4));  // part_o: any float's alignment
     }
     float M = -1e30f;
 #pragma unroll

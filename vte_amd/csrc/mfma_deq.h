@@ -299,10 +299,14 @@ __device__ __forceinline__ void q4_xmin(const half8_t (&bx)[8][NT], float* xl, X
 // One super-block of MFMA work for NT 16-column activation tiles bx[t][nt]
 // (A operands, k-slot map of the format) against one lane's exact weight
 // operands: acc[nt] += d * sum(w x) [- dmin * sum_j m_j X_j], the sums in fp32
-// over the super-block's 8 k-steps in order.  Every batched kernel goes
-// through these functions, so for a given minimum-term form (XM) a weight
-// row's result depends only on which super-blocks a wave sums (and the order
-// the waves' partials are added), not on the kernel or the number of columns.
+// over the super-block's 8 k-steps in order.  The launches of 17 to 32 columns,
+// the weight-stationary and the streaming kernels go through these functions
+// (one-tile launches through sb_staged, with the same sums; the tiled kernels
+// through mt_loop, which rounds a scaled super-block before it adds it).  So for
+// a given minimum-term form (XM) a weight row's result depends only on which
+// super-blocks a wave sums and the order the waves' partials are added, and the
+// tiled kernels agree bit for bit where each of those waves has at most one
+// super-block (K of at most 2048, or that share of K), not beyond.
 template <int NT, bool XM>
 __device__ __forceinline__ void sb_mfma(const Q6Ops& o, const half8_t (&bx)[8][NT], const XMin<NT, XM>&,
                                         floatx4_t (&acc)[NT]) {

@@ -19,7 +19,9 @@
 // Sums: one C tile per super-block (its eight k-steps in order, then the fp32
 // scales), added to the running sum in super-block order.  That is the order
 // of the kernels that give every super-block of a split its own wave and add
-// the waves in order, so the results have the same bits.
+// the waves in order, so the results have the same bits as theirs; where a wave
+// of theirs sums several super-blocks (a share of K above 2048) it folds them
+// into one fma chain, and the results agree to fp32 rounding.
 #pragma once
 #include "mfma_deq.h"
 
