@@ -117,11 +117,12 @@ long long vte_attn_scratch_floats(int batch, int n_q, int max_splits);
  * vte_attn_out_gemv to combine.  kv_batch_stride 0 with B > 1: every column
  * reads the same cache (prompt tokens of one sequence, each at its own
  * kv_offset); two columns then share each K/V tile load, same results.  Above
- * 64 such columns (counters NULL, out given, 0 < scale <= 1e6) blocks of 64
- * (column, head) rows share K/V tiles: probabilities in two fp16 parts where the
- * other forms take one, so the results differ from theirs by the fp16 rounding
- * of the probabilities (3e-4 of a result's norm) and are the closer ones; their
- * bits do not depend on max_splits * split from 1024 rows (and 8 splits) on.
+ * 64 such columns and 96 (column, head) rows (counters NULL, out given,
+ * 0 < scale <= 1e6) blocks of 64 rows share K/V tiles: probabilities in two
+ * fp16 parts where the other forms take one, so the results differ from theirs
+ * by the fp16 rounding of the probabilities (3e-4 of a result's norm) and are
+ * the closer ones; their bits do not depend on max_splits * split from 1024
+ * rows (and 8 splits) on.
  * Replaces: SplitKVAttentionDispatcher launches (vte/core/split_kv_attention.py:187-217),
  *           flash_attention_split_kv_partial_kernel (flash_attention_split_kv_partial.hip.template:31-120),
  *           flash_attention_split_kv_reduce_kernel (flash_attention_split_kv_reduce.hip.template:14-67). */

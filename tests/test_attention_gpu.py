@@ -408,3 +408,21 @@ def test_prompt_chunk_bits_do_not_depend_on_the_capacity(hip, K, B, start, n_q, 
         if rows >= 1024:
             assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), rows
         assert rel_l2(got, ref) <= 2e-6, rows  # two parts of a probability: 2^-21, and fp32 sums
+
+
+@pytest.mark.parametrize("B,same", [(96, True), (97, False)])
+def test_prompt_chunk_of_few_rows(hip, K, B, same):
+    """Up to 96 (column, head) rows keep the two-column blocks and their bits; one more takes the 64-row blocks."""
+    import os
+    rng = np.random.default_rng(B)
+    q = rng.standard_normal((B, 1, D)).astype(np.float32)
+    kc, vc = (rng.standard_normal((1200, 1, D)).astype(np.float16) for _ in range(2))
+    off = np.arange(1000, 1000 + B, dtype=np.int32)
+    got = _prompt_run(hip, K, q, kc, vc, off, 1, 1)
+    os.environ["VTE_ATT_QC"] = "0"
+    try:
+        one = _prompt_run(hip, K, q, kc, vc, off, 1, 1)
+    finally:
+        del os.environ["VTE_ATT_QC"]
+    assert np.array_equal(got.view(np.uint32), one.view(np.uint32)) == same
+    assert rel_l2(got, one) <= TOL

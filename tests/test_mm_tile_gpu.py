@@ -60,6 +60,7 @@ def test_ffn_in_tiled(hip, K, k, ffn, B):
                                               ("q6_k", 8960, 1500, 200, 7), ("q4_k", 256, 9000, 512, 1)])
 def test_splitk_tiled(hip, K, fmt, k, n, M, splits):
     """Split-K partial sums of the tiled form: the bits of the 32-column launches."""
+    import os
     rng = np.random.default_rng(k + M)
     raw = syn.random_matrix(fmt, rng, n, k, balanced=True)
     x = rng.standard_normal((M, k)).astype(np.float16)

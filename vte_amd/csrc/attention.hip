@@ -483,10 +483,12 @@ static bool getenv_off_att(const char* name) {
 // columns per K/V read.  After 1536 rows, 512 / 128 / 80 columns 77.8 / 27.4 /
 // 21.2 -> 27.2 / 14.5 / 13.2 us (at start 0 32.5 / 13.7 / 10.6 -> 16.8 / 8.6 /
 // 8.2); at 64 columns and fewer the two-column blocks, which give the bits of the
-// decode path.  A scale past 1e6 could overflow the masked rows' exponents.
-static bool prompt_form(int B, int kv_batch_stride, float scale, const void* out, const int* counters) {
-    return kv_batch_stride == 0 && B > 64 && counters == nullptr && out != nullptr && scale > 0.f && scale <= 1e6f &&
-           !getenv_off_att("VTE_ATT_QC");
+// decode path, and at no more than a block and a half of rows (one head, 80
+// columns after 7000 rows 21.4 us against 23.7, 112 columns the other way).  A
+// scale past 1e6 could overflow the masked rows' exponents.
+static bool prompt_form(int B, int n_q, int kv_batch_stride, float scale, const void* out, const int* counters) {
+    return kv_batch_stride == 0 && B > 64 && (long long)B * n_q > AP_ROWS * 3 / 2 && counters == nullptr &&
+           out != nullptr && scale > 0.f && scale <= 1e6f && !getenv_off_att("VTE_ATT_QC");
 }
 
 template <typename TQ, typename TO>
@@ -516,7 +518,7 @@ template <typename TQ, typename TO>
 hipError_t attn_split_kv(const void* q, const void* k_cache, const void* v_cache, float* part_m, float* part_l,
                          float* part_o, void* out, int B, int n_q, int n_kv, float scale, const int* kv_offset,
                          int kv_batch_stride, int split, int max_splits, int* counters, hipStream_t st) {
-    if (prompt_form(B, kv_batch_stride, scale, out, counters))
+    if (prompt_form(B, n_q, kv_batch_stride, scale, out, counters))
         return attn_prompt<TQ, TO>(q, k_cache, v_cache, part_m, part_l, part_o, out, B, n_q, n_kv, scale, kv_offset,
                                    (int)std::min(2147483647LL, (long long)max_splits * split), max_splits, st);
     dim3 g1(max_splits, n_kv, B), b1(256);
