@@ -427,19 +427,30 @@ static int mm_env(const char* name, int dflt) {
 
 // Launch form of a batch of B columns, `tiles` 32-row tiles in all.  Above 32
 // columns at K = 6 super-blocks the weight-stationary form, whose six waves each
-// take a super-block, while its column groups are few: q/k/v up to 1.5 blocks of
-// the tiled form (128 rows x 32 columns) per CU, gate/up up to half a block (its
-// blocks hold twice the rows).  q/k/v of 2048 rows, 512 / 768 / 1024 columns 17.4 /
-// 22.2 / 29.8 us against 20.0 / 25.1 / 28.5 tiled, of 4608 rows, 256 / 384 columns
-// 22.1 / 26.8 against 23.9 / 25.4; gate/up of 2 x 2000 rows, 128 / 160 / 384 columns
-// 9.8 / 13.6 / 18.2 against 12.9 / 12.8 / 17.6, of 2 x 8960, 64 columns 24.3 against
-// 17.4.  Both forms give the same bits there.  Other K as in mt_beats_launches.
+// take a super-block, against the tiled one (the same bits there).  Its time goes
+// with the 16-column steps that a CU takes one after another in blocks of 64 rows
+// (a further round of blocks, which decodes its weights again, costs one more):
+// gate/up 9.5 / 11.1 / 13.8 / 16.3 / 18.2 us for 2 / 3 / 4 / 5 / 6 steps, where the
+// tiled form takes 12.8-14.2 with up to a block (of 128 rows x 32 columns) per CU and
+// 17.7-18.9 with up to two; q/k/v 12.4 / 17.1 / 21.8 / 26.8 for 2 / 4 / 6 / 8 against
+// 20-21, 24-25 and 28.5 beyond with Q6_K rows, 16.5 and 21.5 without.  Up to 128
+// columns q/k/v takes smaller blocks (8.5 us at 2048 rows, where the tiled form
+// takes 19), while the tiled form would not fill the chip.  Other K as in
+// mt_beats_launches.
 // VTE_MM_WS=0 selects the 32-column launches for every batch.
 enum MmForm { MM_COLS32, MM_WS, MM_TILED };
-static MmForm mm_form(int B, int tiles, int K, bool swiglu) {
+static MmForm mm_form(int B, int tiles, int K, bool swiglu, bool q6) {
     if (B <= 32 || mm_env("VTE_MM_WS", 1) == 0) return MM_COLS32;
-    const int row_blocks = (tiles + MT_WAVES - 1) / MT_WAVES, cus = device_cus();
-    if (K == 6 * QK_K) return row_blocks * ((B + 31) / 32) <= (swiglu ? cus / 2 : cus + cus / 2) ? MM_WS : MM_TILED;
+    const int row_blocks = (tiles + MT_WAVES - 1) / MT_WAVES, chunks = (B + 31) / 32, cus = device_cus();
+    if (K == 6 * QK_K) {
+        const int ws_tiles = (tiles + 1) / 2, g = ws_column_groups(ws_tiles, B, cus);
+        const int cols = (chunks + g - 1) / g * 32, gy = (B + cols - 1) / cols, rounds = (ws_tiles * gy + cus - 1) / cus;
+        const int full = ((B < cols ? B : cols) + 15) / 16, last = (B - (gy - 1) * cols + 15) / 16;
+        const int steps = (rounds - 1) * (full + 1) + (ws_tiles * (gy - 1) <= cus * (rounds - 1) ? last : full);
+        const bool fills = (long long)row_blocks * chunks > cus;
+        if (!swiglu && B <= 128) return fills ? MM_TILED : MM_WS;
+        return steps <= (q6 ? 5 : 3) + (fills ? 2 : 0) ? MM_WS : MM_TILED;
+    }
     // (the launches' blocks: 24 pairs of gate/up rows, 16 rows of q/k/v; RoPE and
     // the cache writes cost the tiled form more than the small blocks)
     const MtCost cost = swiglu ? MtCost{3.9f, 1.55f, 5.1f, 0.3f, 0.008f} : MtCost{7.1f, 1.98f, 4.0f, 0.2f, 0.0105f};
@@ -532,7 +543,7 @@ hipError_t qkv_mm(const void* xn, const void* wq, const void* q_bias, int fmt_q,
                   int fmt_k, const void* wv, const void* v_bias, int fmt_v, void* q_out, void* k_cache, void* v_cache,
                   const int* kv_offset, int kv_batch_stride, const void* rope_cos, const void* rope_sin, int B, int K,
                   int n_q, int n_kv, hipStream_t st) {
-    const MmForm form = mm_form(B, (n_q + 2 * n_kv) * 4, K, false);
+    const MmForm form = mm_form(B, (n_q + 2 * n_kv) * 4, K, false, fmt_v != 4);
     // weight-stationary: 16, 32 or 64 rows per block up to 64, 128 and more
     // columns (2048 rows; 64 / 128 / 256 columns: 6.7 / 11.6 / 19.7 us with 16 rows,
     // 8.1 / 8.3 / 14.6 with 32, 11.5 / 11.6 / 11.7 with 64)
@@ -566,7 +577,7 @@ hipError_t gate_up_mm(const void* xn, const void* w_gate, const void* w_up, int 
     // 16 gate/up pairs per block (half the blocks of 8, activations read half
     // as often); 24 for 17-32 columns (measured: batch 32 2.26 -> 2.18 ms per
     // step, batch 8-16 slightly slower); 32 in the weight-stationary form
-    const MmForm form = mm_form(B, (ffn + 15) / 16, K, true);
+    const MmForm form = mm_form(B, (ffn + 15) / 16, K, true, false);
     const int RT = form == MM_TILED ? 2 : mm_env("VTE_MM_RT_FFN", form == MM_WS ? 4 : B > 16 ? 3 : 2);
     MmPlan P;
     memset(&P, 0, sizeof(P));
