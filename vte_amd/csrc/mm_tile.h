@@ -332,7 +332,7 @@ static inline int mt_pick_nt(int row_blocks, int splits, int M, int cus) {
 // still takes the super-blocks one after another, against launches that each
 // cost a start and grow with the super-blocks and their columns (and with the
 // rounds of their blocks): both linear, us, fitted to 3060 shapes of 33 to 200
-// columns, where the form picked is at most 1.12 times the other (mean 1.001).
+// columns, where the form picked is at most 1.13 times the other (mean 1.001).
 struct MtCost {
     float tile, tile_sb;                   // tiled: a + b n_sb
     float launch, launch_sb, launch_col;   // launches (c + d n_sb) + e n_sb M
